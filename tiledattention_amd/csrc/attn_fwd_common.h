@@ -123,7 +123,7 @@ __device__ static inline int pp_swz_k(int row) {
 }
 template <int D>
 __device__ static inline int pp_swz_v(int row) {
-  return D == 128 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2);
+  return D >= 128 ? ((row & 3) << 2) : (((row >> 1) & 1) << 2);
 }
 
 // Buffer resource for rows [0, rows) of a row-major tensor with `row_bytes` between rows:

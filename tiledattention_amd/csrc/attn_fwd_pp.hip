@@ -1,5 +1,6 @@
 // SDPA forward for CDNA4 (gfx950), fp32 accumulation, 128 query rows per workgroup:
-// eight waves in a barrier-locked ping-pong.
+// eight waves in a barrier-locked ping-pong.  (Key steps and stages below are those of D <=
+// 160; D = 256 takes steps of 64 keys, 32 a group, see pp_step_keys.)
 //
 // Math: the reference's tiled forward with fp32 accumulation
 // (src/tiledattention/kernels/flash_fwd.py:374-446, unmasked form :533-574): per query row
@@ -39,8 +40,24 @@
 
 namespace ta {
 
-// Stage size of the eight-wave kernel at head dim D: 128 key rows of 2 D bytes.
-constexpr int pp_stage_bytes(int d) { return kPPKeys * 2 * d; }
+// Keys of a workgroup step (half of them per wave group) and bytes of a K or V stage, 2 D
+// bytes a key row, of the eight-wave kernel at head dim D: 128 keys, 64 at D = 256, so that
+// two stages of K and of V take 130 KiB of LDS there.  A cluster is then 16 QK^T and 16 P.V
+// MFMAs as at D = 128, with half the scores a lane, and is bound by its MFMAs and their LDS
+// operands (1 KiB each): bf16 B1 H8 S4096 non-causal 1080 TFLOP/s, causal 188 (four-wave
+// kernel) -> 87 us.
+constexpr int pp_step_keys(int d) { return d == 256 ? kPPKeys / 2 : kPPKeys; }
+constexpr int pp_stage_bytes(int d) { return pp_step_keys(d) * 2 * d; }
+// LDS bytes from one 1 KiB chunk of a K stage to the next: at D = 256 (two rows a chunk) 32
+// more than the chunk, which moves each row pair on by two 16-byte columns.  A b128 read pass
+// covers 16 consecutive rows at one column, eight pairs, whose two rows swap 16-byte columns
+// in twos (physical chunk = logical ^ (row & 1)): 16 distinct columns, and a lane's read
+// addresses along a row are one register plus immediates, where an XOR over 16 rows takes
+// eight.  The registers that saves hold operands read ahead: with them the scheduler keeps
+// the reads four MFMAs in front of their use, without them none (B1 H8 S4096 causal bf16
+// 141 us).
+constexpr int pp_k_chunk(int d) { return d == 256 ? 1024 + 32 : 1024; }
+constexpr int pp_k_stage_bytes(int d) { return pp_stage_bytes(d) / 1024 * pp_k_chunk(d); }
 
 // Partials of split blocks (part_o, part_lse) are written and, by the in-kernel merge,
 // read with agent-scope cache policy (SC1: the form the compiler gives agent-scope atomic
@@ -97,20 +114,21 @@ template <int DT, int D, bool CAUSAL, bool TAIL, bool SPLIT, int TMR = 128, int 
 __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const WorkItem wi, char* lds_k0,
                                                   char* lds_k1, char* lds_v0, char* lds_v1) {
   constexpr int TM = TMR;            // query rows per workgroup
-  constexpr int TK = 128;            // keys per workgroup step (64 per wave group)
+  constexpr int TK = pp_step_keys(D);  // keys per workgroup step
+  constexpr int GK = TK / 2;           // ... per wave group
   // 256 rows (non-causal whole rows): the two groups own different rows, 128 each, and every
   // wave takes all 128 keys of a step (64 MFMAs a cluster, 64 scores a lane).
   constexpr bool R256 = TMR == 256;
   constexpr int NRB = R256 ? 4 : TM / 32;   // 32-row blocks of a group
-  constexpr int NKS = R256 ? 1 : 4 / NRB;   // key slots of a group's 64 keys (1 or 2)
-  constexpr int KB = R256 ? 4 : 2 / NKS;    // 32-key blocks per wave per step
+  constexpr int NKS = R256 ? 1 : 4 / NRB;   // key slots of a group's keys (1 or 2)
+  constexpr int KB = R256 ? 4 : GK / 32 / NKS;  // 32-key blocks per wave per step
   // A stage holds 128 key rows: the first DA columns of each row in a main part (rows of
   // 2 DA bytes; DA = 128 at D = 160, 64 at D = 96, D otherwise), the rest (32 columns at
   // D = 96 and 160) in a tail part of 64-byte rows behind it, so both parts have
   // power-of-two rows.
-  constexpr int DA = D > 128 ? 128 : D == 96 ? 64 : D;
+  constexpr int DA = D == 160 ? 128 : D == 96 ? 64 : D;
   constexpr int DT2 = D - DA;        // tail columns
-  static_assert(DT2 == 0 || DT2 == 32, "head dims 64, 96, 128 and 160");
+  static_assert(DT2 == 0 || DT2 == 32, "head dims 64, 96, 128, 160 and 256");
   constexpr int DK = D / 16;         // k-steps of the QK^T product
   constexpr int DKA = DA / 16;       // ... whose K operand is in the main part
   constexpr int DB = D / 32;         // 32-wide d blocks of O
@@ -125,8 +143,9 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   constexpr int NLDT = DT2 ? 1 : 0;  // tail loads (a group's 64 tail rows are 4 KiB)
   constexpr int NLDS = NLD + NLDT;   // loads per wave per tensor per step (own half)
   static_assert(STAGE_A % (8 * 1024) == 0, "stage must split over the eight waves");
-  static_assert(TK == kPPKeys && (TM == kPPRows || TM == 64 || R256),
-                "steps of 128 keys, blocks of 64, 128 or 256 rows");
+  static_assert(TM == kPPRows || TM == 64 || R256, "blocks of 64, 128 or 256 rows");
+  static_assert(D != 256 || (TM == kPPRows && !SPLIT && LOWP_TN == 0),
+                "D = 256: whole rows, 128 a block, fp32 accumulation");
   static_assert(!R256 || (!CAUSAL && !SPLIT && LOWP_TN == 0 && (D == 64 || D == 128)),
                 "256-row blocks: non-causal whole rows, fp32 accumulation, D 64 or 128");
   static_assert(TM != 64 || D == 64 || D == 96 || D == 128 || D == 160, "64-row blocks: D 64, 96, 128 or 160");
@@ -149,7 +168,7 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   // 5 measured slower).  The other kernels leave it to the compiler (see barrier below).
   constexpr int kLateMfma = TM == 128 && LOWP ? 3 : 0;
 
-  static_assert(STAGE == pp_stage_bytes(D), "stage layout");
+  static_assert(STAGE == pp_stage_bytes(D) && (D != 256 || KB == 1), "stage layout");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -192,7 +211,7 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   // block needs.
   const int t_end = SPLIT ? wi.t_end : ((CAUSAL ? min(S, q0 + TM) : S) + TK - 1) / TK;
   const int wave_kv_end = CAUSAL ? min(S, wq0 + 32) : S;
-  const int gkoff = 64 * grp;              // the group's keys in a step: [TK t + gkoff, + 64)
+  const int gkoff = GK * grp;              // the group's keys in a step: [TK t + gkoff, + GK)
   const int koff = R256 ? 0 : gkoff + 32 * KB * ks;   // this wave's: [TK t + koff, + 32 KB)
 
   // ---- staging: HBM -> LDS directly -------------------------------------------------
@@ -215,7 +234,7 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   // here spans less than 2^31 bytes, so it reads zero (and the per-load row steps added
   // below stay far from 2^32).
   constexpr int kZeroChunk = INT32_MIN;
-  const int lck = ld_pc ^ pp_swz_k<DA>(ld_row);
+  const int lck = D == 256 ? ld_pc ^ (ld_row & 1) : ld_pc ^ pp_swz_k<DA>(ld_row);
   const int lcv = ld_pc ^ pp_swz_v<DA>(ld_row);
   const int kvo = 8 * lck < d_real ? ld_row * k_rb + (lck << 4) : kZeroChunk;
   const int vvo = 8 * lcv < d_real ? ld_row * v_rb + (lcv << 4) : kZeroChunk;
@@ -233,16 +252,20 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   const int q_rb = (int)p.q_ss * 2;
   const int qvo = 8 * lck < d_real ? ld_row * q_rb + (lck << 4) : kZeroChunk;
   const int tqvo = DA + 8 * tl_lck < d_real ? tl_row * q_rb + 2 * DA + (tl_lck << 4) : kZeroChunk;
-  auto dma = [&](const uint16_t* gbase, int64_t row_stride, int rb, int vo, int tvo, int t,
-                 char* stage) {
+  // A chunk's row step from the wave's first goes into the per-lane offset, or at D = 256,
+  // where registers are short, into the load's scalar offset (which the range check includes).
+  constexpr bool kScalarStep = D == 256;
+  constexpr int KCH = pp_k_chunk(D);
+  auto dma = [&](const uint16_t* gbase, int64_t row_stride, int rb, int vo, int tvo, int t, char* stage,
+                 int chunk_bytes) {
     const int row0 = t * TK;
     const int rows = t < t_end ? S - row0 : 0;
     const __amdgpu_buffer_rsrc_t r = row_rsrc(gbase + (int64_t)row0 * row_stride, rows, rb);
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          r, (__attribute__((address_space(3))) void*)(stage + (ld_g0 + LS * i) * 1024), 16,
-          vo + i * LS * RPL * rb, 0, 0, 0);
+          r, (__attribute__((address_space(3))) void*)(stage + (ld_g0 + LS * i) * chunk_bytes), 16,
+          kScalarStep ? vo : vo + i * LS * RPL * rb, kScalarStep ? i * LS * RPL * rb : 0, 0, 0);
     }
     if constexpr (NLDT != 0) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -250,6 +273,9 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
           16, tvo, 0, 0, 0);
     }
   };
+  // This wave's share of K or V of step t into a stage.
+  auto dma_k = [&](int t, char* stage) { dma(kp, p.k_ss, k_rb, kvo, tkvo, t, stage, KCH); };
+  auto dma_v = [&](int t, char* stage) { dma(vp, p.v_ss, v_rb, vvo, tvvo, t, stage, 1024); };
   // The Q tile into `stage` in a K stage's layout, each group loading its half of the rows;
   // rows past S are outside the resource and read as zero.  Against per-lane global loads
   // of each wave's own rows (both groups loading the same rows, 32 rows an instruction)
@@ -278,7 +304,8 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   // that is byte (koff + l32) * RB + (32 * (m >> 1) + 16 * (hl ^ (m & 1))) ^ (32 kk), plus
   // 32 * bk * RB.
   const int mk = pp_swz_k<DA>(l32);
-  const int k_rd = (koff + l32) * RB + 32 * (mk >> 1) + 16 * (hl ^ (mk & 1));
+  const int k_rd = D == 256 ? ((koff + l32) >> 1) * KCH + (l32 & 1) * RB + 16 * (hl ^ (l32 & 1))
+                            : (koff + l32) * RB + 32 * (mk >> 1) + 16 * (hl ^ (mk & 1));
   // K tail (k-steps DKA, DKA + 1): logical chunk 2 (kk - DKA) + hl of tail row
   // koff + 32 bk + l32, physical chunk logical ^ ((l32 >> 2) & 3): byte
   // kt_rd ^ (32 (kk - DKA)) of the tail part, plus 32 * bk * RBT.
@@ -313,6 +340,11 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   f32x16 s[KB];        // S^T blocks of the step whose softmax comes next
   uint32_t pk[KB][8];  // packed P of the step whose P.V comes next
 
+  // Byte of k-step kk in this lane's K row, and of d block db in its V row.  (D = 256: V's
+  // swizzle stays within 256 bytes, so the upper half of a row is an immediate.)
+  auto k_col = [&](int kk) { return D == 256 ? k_rd + 32 * kk : k_rd ^ (32 * kk); };
+  auto v_col = [&](int db) { return D == 256 ? (v_rd ^ (64 * (db & 3))) + 256 * (db >> 2) : v_rd ^ (64 * db); };
+
   // S^T = K Q^T of a step from stage `kst`, every block (blocks holding no key the wave
   // needs are masked whole by the softmax).
   auto qk = [&](const char* kst) {
@@ -320,7 +352,7 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
     for (int kk = 0; kk < DK; ++kk) {
 #pragma unroll
       for (int bk = 0; bk < KB; ++bk) {
-        const char* ap = kk < DKA ? kst + bk * 32 * RB + (k_rd ^ (32 * kk))
+        const char* ap = kk < DKA ? kst + bk * 32 * RB + k_col(kk)
                                   : kst + STAGE_A + bk * 32 * RBT + (kt_rd ^ (32 * (kk - DKA)));
         const u32x4 a = *(const u32x4*)ap;
         s[bk] = DTy::mfma(a, qf[kk], kk == 0 ? f32x16{} : s[bk]);
@@ -341,7 +373,7 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
           const int rbd = db < DBA ? RB : RBT;  // row bytes of the part holding d block db
-          const char* a0p = db < DBA ? vst + (v_rd ^ (64 * db)) + (32 * bk + 16 * kc) * RB
+          const char* a0p = db < DBA ? vst + v_col(db) + (32 * bk + 16 * kc) * RB
                                      : vst + STAGE_A + vt_rd + (32 * bk + 16 * kc) * RBT;
           s16x4 r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)a0p);
           s16x4 r1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(a0p + 8 * rbd));
@@ -602,9 +634,12 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   // landed, and the latencies of all four overlap.  After the barrier every wave reads its
   // Q fragment from lds_v1.  K_1 and V_0 are waited for at the end of the group's first
   // softmax cluster, like the loads of every MFMA cluster.
+  // (256-row blocks and D = 256 read Q straight into registers: their Q tile is 64 KiB,
+  // twice the free stage.)
   static_assert(2 * NLDS < 16, "vmcnt field");
-  dma(kp, p.k_ss, k_rb, kvo, tkvo, t_beg, lds_k0);
-  if constexpr (R256) {
+  constexpr bool kQDirect = R256 || D == 256;
+  dma_k(t_beg, lds_k0);
+  if constexpr (kQDirect) {
     // Q straight into the B-operand registers: lane l holds row wq0 + l % 32, columns
     // 16 kk + 8 (l / 32) .. + 8 (the layout the LDS read below produces); rows past S and
     // columns past d_real are zero.  Counted by vmcnt before K_1 and V_0.
@@ -617,15 +652,15 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   } else if (TM == 128 || grp == 0) {
     dma_q(lds_v1);  // 64-row blocks: group 0's chunks hold every row
   }
-  dma(kp, p.k_ss, k_rb, kvo, tkvo, t_beg + 1, lds_k1);
-  dma(vp, p.v_ss, v_rb, vvo, tvvo, t_beg, lds_v0);
+  dma_k(t_beg + 1, lds_k1);
+  dma_v(t_beg, lds_v0);
   // R256: every prologue load, since the first MFMA cluster of each group reads K_1 and
   // V_0 shares loaded by the other group's waves.
   __builtin_amdgcn_s_waitcnt(R256 ? 0x0F70 : 0x0F70 | (2 * NLDS));
   barrier();
   // Q fragment from lds_v1 (rows 32 wr + l32, read like a K operand); lds_v1 receives V_1
   // only in the first MFMA cluster, at least two barriers later.
-  if constexpr (!R256) {
+  if constexpr (!kQDirect) {
     const int qr = 32 * rb + l32;
 #pragma unroll
     for (int kk = 0; kk < DK; ++kk) {
@@ -660,8 +695,8 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
     // end of its MFMA cluster, so both shares have landed before group 0 reads the stages.
     constexpr bool loads_in_softmax = R256 && decltype(g1_tag)::value;
     if constexpr (loads_in_softmax) {
-      dma(kp, p.k_ss, k_rb, kvo, tkvo, t + 2, k_cur);
-      dma(vp, p.v_ss, v_rb, vvo, tvvo, t + 1, v_nxt);
+      dma_k(t + 2, k_cur);
+      dma_v(t + 1, v_nxt);
     }
     softmax(t, par_tag);
     if constexpr (!loads_in_softmax) wait_dma();  // this wave's K_{t+1} and V_t loads (one cluster ago)
@@ -680,8 +715,8 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
       mfma_cluster_order(0);
       wait_dma();
     } else {
-      dma(kp, p.k_ss, k_rb, kvo, tkvo, t + 2, k_cur);
-      dma(vp, p.v_ss, v_rb, vvo, tvvo, t + 1, v_nxt);
+      dma_k(t + 2, k_cur);
+      dma_v(t + 1, v_nxt);
       mfma_cluster_order(2 * NLDS);
     }
     if constexpr (kPrioMfma) __builtin_amdgcn_s_setprio(0);
@@ -746,33 +781,60 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   // of lds_v0; the merged tile is staged in lds_v1 for row-contiguous stores.
   auto merge_half = [&](auto lo_tag) {
     constexpr int LO = decltype(lo_tag)::value;
+    // This lane, its row and its half.  At D = 256, where O and Q take 192 of a lane's 256
+    // registers, the lane id is read again here: the one the prologue used would be spilled
+    // across the key loop.
+    const int ln = D == 256 ? __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)) : lane;
+    const int lr = D == 256 ? ln & 31 : l32;
+    const int lh = D == 256 ? ln >> 5 : hl;
+    const int mq = wq0 + lr;
     constexpr int NB = DB / 2;
     constexpr int RGN = NB * 16 * 64 * 4;  // bytes a wave sends
-    static_assert(4 * RGN <= STAGE, "a group's exchange regions fit one stage");
+    // D = 256: a group sends 64 KiB, from a K and a V stage (blocks NBS .. NB - 1 from the V
+    // stage), so all four stages are taken and (m, l) go first, through lds_v0.
+    constexpr bool kTwo = 4 * RGN > STAGE;
+    constexpr int NBS = kTwo ? NB / 2 : NB;      // blocks sent from one stage
+    constexpr int RGS = NBS * 16 * 64 * 4;       // bytes a wave sends from one stage
+    static_assert(4 * RGS <= STAGE, "a group's exchange regions fit its stages");
     constexpr int PLO = LO == 0 ? NB : 0;  // first block the partner merges
-    f32x4* mine = (f32x4*)((grp == 0 ? lds_k0 : lds_k1) + wr * RGN);
-    const f32x4* theirs = (const f32x4*)((grp == 0 ? lds_k1 : lds_k0) + wr * RGN);
+    f32x4* mine = (f32x4*)((grp == 0 ? lds_k0 : lds_k1) + wr * RGS);
+    const f32x4* theirs = (const f32x4*)((grp == 0 ? lds_k1 : lds_k0) + wr * RGS);
+    f32x4* mine_v = (f32x4*)((grp == 0 ? lds_v0 : lds_v1) + wr * RGS);
+    const f32x4* theirs_v = (const f32x4*)((grp == 0 ? lds_v1 : lds_v0) + wr * RGS);
     float* ml = (float*)lds_v0;
+    float m1, l1;
+    if constexpr (kTwo) {
+      ml[(grp * 4 + wr) * 128 + ln] = m_run;
+      ml[(grp * 4 + wr) * 128 + 64 + ln] = l_part;
+      barrier();
+      m1 = ml[((1 - grp) * 4 + wr) * 128 + ln];
+      l1 = ml[((1 - grp) * 4 + wr) * 128 + 64 + ln];
+      barrier();
+    }
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int db = PLO + b;
-        mine[(b * 4 + g) * 64 + lane] =
+        (b < NBS ? mine : mine_v)[(b % NBS * 4 + g) * 64 + ln] =
             f32x4{o_acc[db][4 * g], o_acc[db][4 * g + 1], o_acc[db][4 * g + 2], o_acc[db][4 * g + 3]};
       }
     }
-    ml[(grp * 4 + wr) * 128 + lane] = m_run;
-    ml[(grp * 4 + wr) * 128 + 64 + lane] = l_part;
+    if constexpr (!kTwo) {
+      ml[(grp * 4 + wr) * 128 + ln] = m_run;
+      ml[(grp * 4 + wr) * 128 + 64 + ln] = l_part;
+    }
     barrier();
     f32x4 x1[NB][4];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) x1[b][g] = theirs[(b * 4 + g) * 64 + lane];
+      for (int g = 0; g < 4; ++g) x1[b][g] = (b < NBS ? theirs : theirs_v)[(b % NBS * 4 + g) * 64 + ln];
     }
-    const float m1 = ml[((1 - grp) * 4 + wr) * 128 + lane];
-    const float l1 = ml[((1 - grp) * 4 + wr) * 128 + 64 + lane];
+    if constexpr (!kTwo) {
+      m1 = ml[((1 - grp) * 4 + wr) * 128 + ln];
+      l1 = ml[((1 - grp) * 4 + wr) * 128 + 64 + ln];
+    }
     __builtin_amdgcn_sched_barrier(0);
     const float m = vmax(m_run, m1);
     const float a0 = fast_exp2((m_run - m) * c);
@@ -800,48 +862,50 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
     if (SPLIT && slot >= 0) {
       // One chunk of a split block: its output normalised by its own l, in fp32, and
       // log2 of its softmax denominator in units of the scaled scores, m c + log2(l).
-      if (TAIL && my_q >= S) return;
-      float* prow = p.part_o + ((int64_t)slot * TM + (my_q - q0)) * D;
+      if (TAIL && mq >= S) return;
+      float* prow = p.part_o + ((int64_t)slot * TM + (mq - q0)) * D;
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) store_partial(p, prow + 32 * (LO + b) + 8 * g + 4 * hl, merged(b, g));
+        for (int g = 0; g < 4; ++g) store_partial(p, prow + 32 * (LO + b) + 8 * g + 4 * lh, merged(b, g));
       }
-      if (grp == 0 && hl == 0) store_partial(p, p.part_lse + (int64_t)slot * TM + (my_q - q0), m * c + fast_log2(l_tot));
+      if (grp == 0 && lh == 0) store_partial(p, p.part_lse + (int64_t)slot * TM + (mq - q0), m * c + fast_log2(l_tot));
       return;
     }
     // Whole-row kernels at D = 128, and causal ones at D = 64, stage the wave's 32 rows x
     // D/2 columns in lds_v1 (16-byte chunks swizzled with the row's low bits, CH a row) so
     // each store writes 16 bytes a lane, CH lanes a row; the non-causal D = 64 kernels (two
     // workgroups per CU) store 8 bytes a lane directly.
-    constexpr bool kStageOut = !SPLIT && (D == 128 || (D == 64 && CAUSAL));
+    constexpr bool kStageOut = !SPLIT && (D == 128 || D == 256 || (D == 64 && CAUSAL));
     if constexpr (kStageOut) {
       constexpr int CH = 4 * NB;           // 16-byte chunks per staged row (D/2 columns)
       constexpr int RPI = 64 / CH;         // rows per store instruction
       constexpr int SWZ = CH - 1;
-      char* ob = lds_v1 + (grp * 4 + wr) * (32 * CH * 16);
+      // (D = 256: over the values read from the partner, which only this wave reads.)
+      char* ob = kTwo ? (char*)theirs : lds_v1 + (grp * 4 + wr) * (32 * CH * 16);
+      if constexpr (kTwo) asm volatile("" ::: "memory");
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const f32x4 o4 = merged(b, g);
           const int ch = 4 * b + g;
-          *(u32x2*)(ob + l32 * (CH * 16) + 16 * (ch ^ (l32 & SWZ)) + 8 * hl) =
+          *(u32x2*)(ob + lr * (CH * 16) + 16 * (ch ^ (lr & SWZ)) + 8 * lh) =
               u32x2{DTy::pack(o4[0], o4[1]), DTy::pack(o4[2], o4[3])};
         }
       }
       asm volatile("" ::: "memory");
-      const int ch = lane % CH;
+      const int ch = ln % CH;
 #pragma unroll
       for (int i = 0; i < 32 / RPI; ++i) {
-        const int row = RPI * i + lane / CH;
+        const int row = RPI * i + ln / CH;
         const u32x4 v = *(const u32x4*)(ob + row * (CH * 16) + 16 * (ch ^ (row & SWZ)));
         const int q = wq0 + row;
         const int col = 32 * LO + 8 * ch;
         if ((!TAIL || q < S) && col < d_real) {
           // D = 128: non-temporal stores (C3 S = 4096 / 8192 -0.9 / -0.6 %, C4 unchanged);
           // at D = 64, and on the other store paths, they measured slower.
-          if constexpr (D == 128) {
+          if constexpr (D >= 128) {
             __builtin_nontemporal_store(v, (u32x4*)(op + (int64_t)q * p.o_ss + col));
           } else {
             *(u32x4*)(op + (int64_t)q * p.o_ss + col) = v;
@@ -850,14 +914,14 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
       }
       return;
     }
-    if (TAIL && my_q >= S) return;
-    uint16_t* orow = op + (int64_t)my_q * p.o_ss;
+    if (TAIL && mq >= S) return;
+    uint16_t* orow = op + (int64_t)mq * p.o_ss;
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const f32x4 o4 = merged(b, g);
-        const int d = 32 * (LO + b) + 8 * g + 4 * hl;
+        const int d = 32 * (LO + b) + 8 * g + 4 * lh;
         if (d < d_real) *(u32x2*)(orow + d) = u32x2{DTy::pack(o4[0], o4[1]), DTy::pack(o4[2], o4[3])};
       }
     }
@@ -988,7 +1052,7 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   // Group 1 leaves (m, l, O^T) in LDS; group 0 merges and writes O.
   float* xo = (float*)((wr < 2 ? lds_k0 : lds_k1) + (wr & 1) * (STAGE / 2));
   float* xml = (float*)lds_v0 + wr * 128;
-  static_assert(DB * 16 * 64 * 4 <= STAGE / 2, "merge buffer must fit half a stage");
+  static_assert(DB % 2 == 0 || DB * 16 * 64 * 4 <= STAGE / 2, "merge buffer must fit half a stage");
   if (grp == 1) {
 #pragma unroll
     for (int db = 0; db < DB; ++db) {
@@ -1153,8 +1217,8 @@ __device__ __forceinline__ void attn_fwd_pp_body(const FwdParams& p) {
   // One array per (tensor, stage): the stage of every access is a compile-time constant
   // (the key loop is unrolled by two), so the compiler can tell the loads in flight into
   // one stage from the reads of the other and does not wait on the former for the latter.
-  __shared__ __attribute__((aligned(1024))) char lds_k0[STAGE];
-  __shared__ __attribute__((aligned(1024))) char lds_k1[STAGE];
+  __shared__ __attribute__((aligned(1024))) char lds_k0[pp_k_stage_bytes(D)];
+  __shared__ __attribute__((aligned(1024))) char lds_k1[pp_k_stage_bytes(D)];
   __shared__ __attribute__((aligned(1024))) char lds_v0[STAGE];
   __shared__ __attribute__((aligned(1024))) char lds_v1[STAGE];
   // In-kernel merge: whether this workgroup arrived last at its block, in the last word of
@@ -1365,12 +1429,14 @@ __device__ unsigned ta_merge_counters[ta::kMergeRegions * ta::kMergeRegionCounte
 // next, lighter tile as its heavy one ends (two resident from the start measured 5 % slower
 // on B1 H8 S8192), and so do the split kernels, the residency the split planner models.
 #define TA_PP_WAVES(D, C) ((D) == 64 && (C) == 0 ? 4 : 2)
-#define TA_PP_DEFINE(DTN, DT, D, C, T)                                                    \
+#define TA_PP_WHOLE_DEFINE(DTN, DT, D, C, T)                                              \
   extern "C" __global__ void __launch_bounds__(512)                                       \
       __attribute__((amdgpu_waves_per_eu(TA_PP_WAVES(D, C), TA_PP_WAVES(D, C))))           \
       ta_fwd_pp_##DTN##_d##D##_c##C##_t##T(ta::FwdParams p) {                              \
     ta::attn_fwd_pp_body<DT, D, (C != 0), (T != 0), false, false>(p);                     \
-  }                                                                                       \
+  }
+#define TA_PP_DEFINE(DTN, DT, D, C, T)                                                    \
+  TA_PP_WHOLE_DEFINE(DTN, DT, D, C, T)                                                    \
   extern "C" __global__ void __launch_bounds__(512)                                       \
       __attribute__((amdgpu_waves_per_eu(2, 2)))                                          \
       ta_fwd_pp_split_##DTN##_d##D##_c##C##_t##T(ta::FwdParams p) {                        \
@@ -1481,6 +1547,13 @@ TA_PP_DEFINE_CT(bf16, 1, 64)
 TA_PP_DEFINE_CT(bf16, 1, 96)
 TA_PP_DEFINE_CT(bf16, 1, 128)
 TA_PP_DEFINE_CT(bf16, 1, 160)
+#define TA_PP_WHOLE_DEFINE_CT(DTN, DT, D) \
+  TA_PP_WHOLE_DEFINE(DTN, DT, D, 0, 0)    \
+  TA_PP_WHOLE_DEFINE(DTN, DT, D, 0, 1)    \
+  TA_PP_WHOLE_DEFINE(DTN, DT, D, 1, 0)    \
+  TA_PP_WHOLE_DEFINE(DTN, DT, D, 1, 1)
+TA_PP_WHOLE_DEFINE_CT(f16, 0, 256)
+TA_PP_WHOLE_DEFINE_CT(bf16, 1, 256)
 TA_PP_PAIR_DEFINE(f16, 0, 64, 0)
 TA_PP_PAIR_DEFINE(f16, 0, 64, 1)
 TA_PP_PAIR_DEFINE(f16, 0, 96, 0)

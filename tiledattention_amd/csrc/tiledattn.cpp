@@ -631,6 +631,25 @@ bool use_rows256(const ta_fwd_args* a, int64_t n_bh, int ncu) {
   return 2 * rounds256 <= rounds128;
 }
 
+// Whether a whole-row launch at D = 256 runs the eight-wave kernel (ta_fwd_pp_*_d256_*; steps
+// of 64 keys): fp32 accumulation, 128-row tiles, rows of more than one key step (bf16, four-wave
+// kernel -> this one: B1 H8 S4096 causal 188 -> 87 us, B1 H2 S512 27.6 -> 18.1, B4 H16 S128
+// 13.3 -> 11.8; at one step they are even, B1 H8 S64 9.7 -> 10.1, B4 H32 S64 9.7 -> 9.5).  One
+// head of at most four blocks stays on the four-wave kernel, the launch that callers of
+// ta_describe_launch have for it; and a grid whose 512-thread workgroups would pass the
+// dispatch packet's 2^32 work-items, which the four-wave kernel's 256 do not.
+bool use_pp_d256(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk) {
+  return a->D == 256 && a->accum == TA_ACC_FP32 && a->tile_m == 128 && a->tile_n == 64 && a->S > 64 &&
+         (n_bh > 1 || n_qblk > 4) && n_bh * n_qblk * 512 <= 0xffffffffLL;
+}
+
+KernelId pp_d256_kernel_id(int dtype, int causal, int tail) {
+  char buf[64];
+  snprintf(buf, sizeof(buf), "ta_fwd_pp_%s_d256_c%d_t%d", dtype == TA_BF16 ? "bf16" : "f16", causal ? 1 : 0,
+           tail ? 1 : 0);
+  return {kPPObject, buf, 512u};
+}
+
 // Whether split key ranges exist for this configuration: the eight-wave kernels with fp32
 // accumulation, 128-row blocks (chunks and the paired split) or 64-row blocks (chunks, each
 // 128-row item of the numbering run as two 64-row halves).
@@ -739,6 +758,9 @@ ta_status plan_launch(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int32_
       pl->tail = t256;
       pl->layout = TA_LAYOUT_ROWS256;
     }
+  } else if (use_pp_d256(a, n_bh, n_qblk)) {
+    // (tile_m divides the aligned variant's S, so its 64-key steps are whole.)
+    pl->main = pp_d256_kernel_id(a->dtype, a->causal, !aligned);
   } else if (eight_wave64(a->tile_m, a->tile_n, a->accum, a->D) && use_wide(a->S, n_bh, a->D, ncu)) {
     // The aligned variant's S (a multiple of 128) is whole 32-row blocks and whole passes of
     // a wave's keys, as its t0 form needs.
@@ -1080,6 +1102,11 @@ ta_status ta_prepare(int32_t device, int32_t dtype, int32_t head_dim, int32_t ti
   if (guard.err != hipSuccess)
     return fail(TA_EHIP, "set device %d: %s", device, hipGetErrorString(guard.err));
   hipFunction_t fn;
+  if (head_dim == 256 && tile_m == 128 && accum == TA_ACC_FP32) {
+    // Most of its grids run another kernel (use_pp_d256): both are loaded.
+    ta_status st = get_function_locked(device, pp_d256_kernel_id(dtype, causal != 0, aligned == 0), &fn);
+    if (st != TA_OK) return st;
+  }
   return get_function_locked(
       device, kernel_id(dtype, head_dim, tile_m, tile_n, causal != 0, aligned == 0, accum), &fn);
 }
