@@ -330,3 +330,37 @@ def test_policy_defaults_run_the_described_kernels(lib):
                                   head_dim=d, compute_units=CU)
         desc = _d(lib, B=b, H=h, S=s, D=d, causal=causal, tile_m=tm, tile_n=tn, sched=sched, dtype=dtype)
         assert (desc.kernel.decode(), desc.layout) == (kernel, layout), (b, h, s, d)
+
+
+# Small-workgroup kernel: 128-row fp32 tiles, more 128-row blocks than CUs, short rows.
+@pytest.mark.parametrize("d,causal,b,s,rows", [
+    (64, False, 32, 128, False), (64, False, 33, 128, True),        # 256 / 264 blocks of 256 CUs
+    (64, False, 24, 512, True), (64, False, 24, 513, False),        # 768 / 960 blocks
+    (64, False, 16, 1024, True), (64, False, 16, 1025, False),      # four blocks a CU
+    (96, False, 8, 1024, True), (96, False, 8, 1025, False),
+    (128, False, 9, 512, True), (128, False, 9, 513, False),
+    (160, False, 8, 768, True), (160, False, 8, 769, False),
+    (64, True, 16, 384, True), (64, True, 16, 512, False),          # 256 pairs: one full round
+    (64, True, 24, 512, True), (64, True, 8, 768, True), (64, True, 8, 1024, False),
+    (64, True, 12, 1024, True), (64, True, 32, 1024, True),         # 384 pairs; 2048 blocks
+    (96, True, 8, 1536, True), (96, True, 8, 1537, False), (96, True, 16, 1536, False),
+    (128, True, 12, 512, True), (128, True, 16, 512, False), (128, True, 8, 640, False),
+    (128, True, 16, 640, True), (128, True, 12, 768, True), (128, True, 32, 768, False),
+    (128, True, 12, 769, False), (160, True, 8, 640, True), (160, True, 8, 641, False),
+])
+def test_small_workgroup_rule(lib, objects, d, causal, b, s, rows):
+    for aligned in (0, 1):
+        desc = _d(lib, B=b, H=8, S=s, D=d, causal=causal, tile_m=128, sched=1, aligned=aligned)
+        assert desc.kernel.decode().startswith("ta_fwd_rows_") is rows, desc.kernel
+        assert desc.kernel + b"\x00" in objects[desc.code_object.decode()]
+        if rows:
+            assert desc.kernel.decode() == f"ta_fwd_rows_bf16_d{d}_c{int(causal)}_t{int(not (aligned and s % 128 == 0))}"
+            assert (desc.grid, desc.block, desc.rows) == (8 * b * -(-s // 128), 256, 128)
+            assert desc.layout == _lib.TA_LAYOUT_WHOLE_ROWS
+    # forced pairs, 64-row tiles and input-dtype accumulation keep their kernels
+    for kw in (dict(sched=3), dict(tile_m=64), dict(accum=_lib.TA_ACC_INPUT)):
+        if d == 96 and "accum" in kw or d == 160 and "accum" in kw:
+            continue
+        args = dict(B=b, H=8, S=s, D=d, causal=causal, tile_m=128, sched=1)
+        args.update(kw)
+        assert not _d(lib, **args).kernel.decode().startswith("ta_fwd_rows_")

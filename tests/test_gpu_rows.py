@@ -1,0 +1,91 @@
+"""The small-workgroup kernel (ta_fwd_rows_*: short rows on grids of more than one 128-row block
+per CU) against the oracle: one row, one key past a tile, one row past a block, whole tiles
+and blocks, rows that end inside a wave, head dims padded in place, every layout, outliers
+that move the running max between tiles, and non-finite keys."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from tests.parity_util import TOL, as_f32, check_close, inputs, oracle_f32, say
+
+pytestmark = pytest.mark.gpu
+
+
+def _on_gpu(t3, layout):
+    import torch
+
+    dev = torch.device("cuda:0")
+    if layout == "packed":  # slices of one [B, S, 3, H, D] projection
+        p = torch.stack([t.transpose(1, 2) for t in t3], dim=2).contiguous().to(dev)
+        return [p[:, :, i].transpose(1, 2) for i in range(3)]
+    if layout == "bshd":
+        return [t.transpose(1, 2).contiguous().to(dev).transpose(1, 2) for t in t3]
+    return [t.to(dev) for t in t3]
+
+
+def _run(t3, causal, layout="bhsd"):
+    import torch
+
+    from tiledattention import sdpa
+    from tiledattention.kernels import flash_fwd
+
+    args = _on_gpu(t3, layout)
+    desc = flash_fwd.describe_call(*args, causal=causal)
+    assert desc["kernel"].startswith("ta_fwd_rows_"), desc
+    say(f"{desc['kernel']} {tuple(args[0].shape)} {layout}")
+    out = sdpa(*args, causal=causal)
+    torch.cuda.synchronize()
+    return as_f32(out)
+
+
+@pytest.mark.parametrize("shape,causal,dtype,layout", [
+    ((33, 8, 1, 64), True, "float16", "bhsd"),
+    ((33, 8, 64, 64), False, "bfloat16", "packed"),
+    ((33, 8, 65, 96), True, "bfloat16", "bshd"),
+    ((33, 8, 128, 160), False, "float16", "bhsd"),   # whole tiles and blocks: no tail masks
+    ((17, 8, 129, 128), False, "float16", "packed"),
+    ((17, 8, 197, 64), False, "float16", "packed"),
+    ((17, 8, 200, 160), True, "bfloat16", "bhsd"),
+    ((17, 8, 256, 96), False, "float16", "packed"),
+    ((17, 8, 256, 64), True, "bfloat16", "bhsd"),
+    ((17, 8, 225, 40), True, "float16", "bhsd"),     # padded in place to 64
+    ((17, 8, 193, 72), False, "bfloat16", "bshd"),   # ... to 96
+    ((17, 8, 250, 112), True, "bfloat16", "packed"), # ... to 128
+    ((17, 8, 161, 136), False, "float16", "bhsd"),   # ... to 160
+    ((17, 8, 150, 100), False, "bfloat16", "bhsd"),  # padded on the host
+])
+def test_rows_against_the_oracle(gpu, shape, causal, dtype, layout):
+    t3 = inputs(shape, dtype, 700 + shape[2] + shape[3])
+    ref = oracle_f32(*t3, causal=causal)
+    check_close(_run(t3, causal, layout), ref, dtype, tol=TOL[dtype], what=f"rows {shape} {layout}")
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_rows_rescale_between_tiles(gpu, d):
+    """Keys whose size grows tile by tile raise each row's max past the rescale threshold."""
+    import torch
+
+    q, k, v = inputs((33, 8, 256, d), "bfloat16", 81 + d)
+    k = (k.float() * torch.linspace(0.1, 12.0, 256)[None, None, :, None]).to(k.dtype)
+    ref = oracle_f32(q, k, v, causal=False)
+    # nearly one-hot rows: P's rounding (u = 2^-8) moves O by up to 3 u max|v|
+    tol = 3 * 2.0 ** -8 * float(v.float().abs().max())
+    check_close(_run((q, k, v), False), ref, "bfloat16", tol=tol, what=f"rows rescale D={d}")
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("-inf")])
+def test_rows_nonfinite_keys(gpu, value):
+    """A NaN key poisons every row of its head; a key whose scores are -inf or +inf by the
+    sign of q's column poisons the rows where they are +inf (inf - inf) and no others."""
+    q, k, v = inputs((33, 8, 150, 64), "bfloat16", 5)
+    k = k.clone()
+    k[0, 1, 3, 7] = value
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = oracle_f32(q, k, v, causal=False)
+    got = _run((q, k, v), False)
+    assert (np.isnan(got) == np.isnan(ref)).all() and np.isnan(ref).any()
+    fin = np.isfinite(ref)
+    assert np.isfinite(got[fin]).all()
+    assert float(np.abs(got[fin] - ref[fin]).max()) <= TOL["bfloat16"]

@@ -35,6 +35,7 @@
 
 #include "attn_fwd_common.h"
 #include "attn_fwd_params.h"
+#include "attn_fwd_rows.h"
 
 namespace ta {
 
@@ -370,3 +371,14 @@ TA_WIDE_DEFINE_CT(f16, 0, 64)
 TA_WIDE_DEFINE_CT(f16, 0, 128)
 TA_WIDE_DEFINE_CT(bf16, 1, 64)
 TA_WIDE_DEFINE_CT(bf16, 1, 128)
+
+// Small-workgroup kernels (attn_fwd_rows.h): four workgroups a CU at D = 64 (128 VGPRs, 32 KiB
+// of LDS), three at D = 96, two at 128 and 160.
+TA_ROWS_DEFINE_CT(f16, 0, 64, 4)
+TA_ROWS_DEFINE_CT(f16, 0, 96, 3)
+TA_ROWS_DEFINE_CT(f16, 0, 128, 2)
+TA_ROWS_DEFINE_CT(f16, 0, 160, 2)
+TA_ROWS_DEFINE_CT(bf16, 1, 64, 4)
+TA_ROWS_DEFINE_CT(bf16, 1, 96, 3)
+TA_ROWS_DEFINE_CT(bf16, 1, 128, 2)
+TA_ROWS_DEFINE_CT(bf16, 1, 160, 2)

@@ -203,25 +203,17 @@ ta_status check_arch_locked(int device) {
   return TA_OK;
 }
 
-// Caller holds g_mu and has made `device` current.
-ta_status get_function_locked(int device, const KernelId& id, hipFunction_t* out) {
-  auto fk = std::make_pair(device, id.name);
-  auto fit = g_funcs.find(fk);
-  if (fit != g_funcs.end()) {
-    *out = fit->second;
-    return TA_OK;
-  }
-  ta_status st = check_arch_locked(device);
-  if (st != TA_OK) return st;
-  auto mk = std::make_pair(device, id.file);
+// Caller holds g_mu and has made `device` current.  The module of a code object file.
+ta_status load_module_locked(int device, const std::string& file, hipModule_t* out) {
+  auto mk = std::make_pair(device, file);
   hipModule_t mod = nullptr;
   auto mit = g_modules.find(mk);
   if (mit == g_modules.end()) {
-    std::string path = (g_dir.empty() ? default_dir() : g_dir) + "/" + id.file;
+    std::string path = (g_dir.empty() ? default_dir() : g_dir) + "/" + file;
     hipError_t e = hipModuleLoad(&mod, path.c_str());
     if (e != hipSuccess)
       return fail(TA_ENOKERNEL, "hipModuleLoad(%s): %s", path.c_str(), hipGetErrorString(e));
-    if (id.file == kPPObject) {
+    if (file == kPPObject) {
       // The merge counters start at zero; every launch leaves them zero.  Zeroed here
       // once per load, synchronously, before any kernel of the module can run.
       hipDeviceptr_t cnt = nullptr;
@@ -246,6 +238,23 @@ ta_status get_function_locked(int device, const KernelId& id, hipFunction_t* out
   } else {
     mod = mit->second;
   }
+  *out = mod;
+  return TA_OK;
+}
+
+// Caller holds g_mu and has made `device` current.
+ta_status get_function_locked(int device, const KernelId& id, hipFunction_t* out) {
+  auto fk = std::make_pair(device, id.name);
+  auto fit = g_funcs.find(fk);
+  if (fit != g_funcs.end()) {
+    *out = fit->second;
+    return TA_OK;
+  }
+  ta_status st = check_arch_locked(device);
+  if (st != TA_OK) return st;
+  hipModule_t mod = nullptr;
+  st = load_module_locked(device, id.file, &mod);
+  if (st != TA_OK) return st;
   hipFunction_t fn = nullptr;
   hipError_t e = hipModuleGetFunction(&fn, mod, id.name.c_str());
   if (e != hipSuccess)
@@ -650,6 +659,46 @@ KernelId pp_d256_kernel_id(int dtype, int causal, int tail) {
   return {kPPObject, buf, 512u};
 }
 
+// Whether a whole-row launch of a 128-row fp32 tile runs the small-workgroup kernel
+// (attn_fwd_rows.h, ta_fwd_rows_*): grids of more than one 128-row block per CU with short
+// rows.  There an eight-wave workgroup's fixed cost (prologue, pipeline fill, merge of its
+// key halves) comes to as much as its few key steps, one workgroup a CU; the small ones,
+// two to four a CU, run one's loads under another's products.  Lines by measurement (bf16,
+// 8-1024 heads, S 48-2048; eight-wave kernel -> this one, us):
+// * at most one block per CU loses (D = 64 S512 64 heads 9.2 -> 9.7, D = 128 S384 64 heads
+//   9.5 -> 11.4): the eight-wave kernel's blocks are twice as fast each;
+// * non-causal: D = 64 up to S = 512 (256 heads 30.8 -> 25.0; S640 96 heads 15.5 -> 15.8), and
+//   1024 from four blocks a CU (128 heads 44.7 -> 40.5); D = 128 up to 512, against its 256-row
+//   blocks (256 heads 51.3 -> 44.3; S640 64 heads 22.6 -> 23.3); D = 96 up to 1024 (64 heads
+//   32.5 -> 32.2; S1536 32 heads 36.8 -> 38.4); D = 160 up to 768 (34.0 -> 32.8; S1024 96 heads
+//   69.7 -> 70.6);
+// * causal, against pairs of blocks (two or more blocks a CU): where the pairs fill one round
+//   of the CUs (85 % or more) only up to S = 384 (D = 64 S512 128 heads 12.8 -> 13.2, D = 128
+//   20.7 -> 21.7; S384 22.6 -> 19 and more); otherwise D = 64 and 96 up to S = 768 (D = 64 S512
+//   192 heads 25.3 -> 18.5), to 1024 past four blocks a CU (256 heads 66.6 -> 57), and to 1536
+//   where the pairs' last round is short (S1536 64 heads, 384 pairs, 38.0 -> 32.4, 512 pairs
+//   S1024 33.6 -> 34.3); D = 128 up to 512, 640 past two blocks a CU (S640 192 heads 48.5 ->
+//   40.0, 64 heads 18.3 -> 20.1) and 768 where the pairs' last round is short (192 heads 61.9
+//   -> 52, 256 heads 65.1 -> 65.6); D = 160, which has no pairs, up to 640 (96 heads 28.4 ->
+//   24.8; S768 35.3 -> 37.1).
+bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
+  if (!eight_wave(a->tile_m, a->tile_n, a->accum, a->D) || a->sched == 3 || ncu <= 0) return false;
+  const int64_t S = a->S, n = n_bh * n_qblk;
+  if (n <= ncu) return false;
+  if (!a->causal) {
+    if (a->D == 64) return S <= 512 || (S <= 1024 && n >= 4 * (int64_t)ncu);
+    return S <= (a->D == 96 ? 1024 : a->D == 128 ? 512 : 768);
+  }
+  if (a->D == 160) return S <= 640;
+  const bool paired = n >= 2 * (int64_t)ncu;
+  const int64_t pairs = n_bh * ((n_qblk + 1) / 2), rounds = (pairs + ncu - 1) / ncu;
+  const bool full = 100 * pairs >= 85 * rounds * ncu;  // the pairs' last round
+  if (S <= 384) return true;
+  if (paired && full && rounds == 1) return false;
+  if (a->D == 128) return S <= 512 || (S <= 640 && paired) || (S <= 768 && paired && !full);
+  return S <= 768 || (S <= 1024 && n > 4 * (int64_t)ncu) || (S <= 1536 && paired && !full);
+}
+
 // Whether split key ranges exist for this configuration: the eight-wave kernels with fp32
 // accumulation, 128-row blocks (chunks and the paired split) or 64-row blocks (chunks, each
 // 128-row item of the numbering run as two 64-row halves).
@@ -742,7 +791,11 @@ ta_status plan_launch(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int32_
   pl->main = kernel_id(a->dtype, (int)a->D, a->tile_m, a->tile_n, a->causal, !aligned, a->accum);
   pl->grid = n_bh * n_qblk;
   pl->rows = a->tile_m;
-  if (eight_wave(a->tile_m, a->tile_n, a->accum, a->D)) {
+  if (use_rows(a, n_bh, n_qblk, ncu)) {
+    char name[64];
+    snprintf(name, sizeof(name), "ta_fwd_rows_%s_d%d_c%d_t%d", dt, (int)a->D, a->causal ? 1 : 0, aligned ? 0 : 1);
+    pl->main = KernelId{kWideObject, name, 256u};
+  } else if (eight_wave(a->tile_m, a->tile_n, a->accum, a->D)) {
     if (a->causal && use_pairs(a, n_bh, n_qblk, ncu)) {
       pl->main = pair_kernel_id(a->dtype, (int)a->D, !aligned);
       pl->grid = n_bh * ((n_qblk + 1) / 2);
@@ -1107,8 +1160,14 @@ ta_status ta_prepare(int32_t device, int32_t dtype, int32_t head_dim, int32_t ti
     ta_status st = get_function_locked(device, pp_d256_kernel_id(dtype, causal != 0, aligned == 0), &fn);
     if (st != TA_OK) return st;
   }
-  return get_function_locked(
+  ta_status st = get_function_locked(
       device, kernel_id(dtype, head_dim, tile_m, tile_n, causal != 0, aligned == 0, accum), &fn);
+  if (st != TA_OK || accum != TA_ACC_FP32 || head_dim > 160) return st;
+  // Short rows run kernels of another code object (use_wide, use_rows): loaded here too, so
+  // that a launch, which may be captured, finds it (a failure is that launch's to report).
+  hipModule_t mod = nullptr;
+  (void)load_module_locked(device, kWideObject, &mod);
+  return TA_OK;
 }
 
 ta_status ta_sdpa_fwd(const ta_fwd_args* a, void* stream) {
