@@ -364,3 +364,22 @@ def test_small_workgroup_rule(lib, objects, d, causal, b, s, rows):
         args = dict(B=b, H=8, S=s, D=d, causal=causal, tile_m=128, sched=1)
         args.update(kw)
         assert not _d(lib, **args).kernel.decode().startswith("ta_fwd_rows_")
+
+
+# The same workgroups with input-dtype accumulation: 128-row tiles, more blocks than CUs.
+@pytest.mark.parametrize("d,tn,causal,b,s,rows", [
+    (64, 64, False, 32, 128, False), (64, 64, False, 33, 128, True), (64, 128, False, 4, 16384, True),
+    (64, 64, True, 8, 1024, True), (64, 64, True, 4, 2048, False), (64, 128, True, 6, 2048, True),
+    (64, 64, True, 6, 3072, False), (64, 64, True, 8, 3072, True), (64, 64, True, 16, 3073, False),
+    (128, 64, False, 2, 4096, True), (128, 64, False, 2, 4097, False), (128, 64, True, 16, 2048, True),
+    (128, 64, True, 16, 2049, False), (128, 128, False, 16, 768, True), (128, 128, False, 16, 769, False),
+    (128, 128, True, 16, 512, True), (128, 128, True, 16, 513, False),
+])
+def test_small_workgroup_rule_input_dtype(lib, objects, d, tn, causal, b, s, rows):
+    desc = _d(lib, B=b, H=8, S=s, D=d, causal=causal, tile_m=128, tile_n=tn, sched=1, accum=_lib.TA_ACC_INPUT)
+    fam = "rowsl" if rows else "ppl"
+    assert desc.kernel.decode() == f"ta_fwd_{fam}_n{tn}_bf16_d{d}_c{int(causal)}_t{int(s % 128 != 0)}"
+    assert desc.kernel + b"\x00" in objects[desc.code_object.decode()]
+    assert (desc.grid, desc.block, desc.rows) == (8 * b * -(-s // 128), 256 if rows else 512, 128)
+    d64 = _d(lib, B=b, H=8, S=s, D=d, causal=causal, tile_m=64, tile_n=tn, sched=1, accum=_lib.TA_ACC_INPUT)
+    assert d64.kernel.decode().startswith("ta_fwd_ppl64_")

@@ -89,3 +89,35 @@ def test_rows_nonfinite_keys(gpu, value):
     fin = np.isfinite(ref)
     assert np.isfinite(got[fin]).all()
     assert float(np.abs(got[fin] - ref[fin]).max()) <= TOL["bfloat16"]
+
+
+@pytest.mark.parametrize("shape,causal,dtype,tile_n,layout", [
+    ((33, 8, 64, 64), False, "float16", 64, "packed"),     # one tile: the second slice empty
+    ((33, 8, 65, 128), True, "bfloat16", 64, "bhsd"),
+    ((33, 8, 128, 128), False, "float16", 128, "bhsd"),    # whole tiles and blocks
+    ((17, 8, 200, 64), True, "bfloat16", 128, "bshd"),
+    ((17, 8, 384, 64), False, "bfloat16", 64, "bhsd"),
+    ((17, 8, 321, 40), False, "float16", 64, "bhsd"),      # padded in place to 64
+    ((17, 8, 250, 112), True, "float16", 128, "packed"),   # ... to 128
+])
+def test_rows_input_dtype_accumulation(gpu, shape, causal, dtype, tile_n, layout):
+    """Against the oracle's restatement of the rounding sequence at the fp32 tolerance, as the
+    eight-wave kernel's results are (each tile's rounding is at most half an ulp of a partial
+    sum whose weights add up to at most the row's)."""
+    import torch
+
+    from oracle import oracle as O
+    from tiledattention import torch_op  # noqa: F401  (registers the operator)
+    from tiledattention.kernels import flash_fwd
+
+    t3 = inputs(shape, dtype, 900 + shape[2])
+    code = O.FP16 if dtype == "float16" else O.BF16
+    bits = O.flash_tiled(*(O.to_bits(t) for t in t3), code, causal=causal, tile_m=128, tile_n=tile_n, accum_lowp=True)
+    ref = O.upcast(bits, code)
+    args = _on_gpu(t3, layout)
+    desc = flash_fwd.describe_call(*args, causal=causal, tile=(128, tile_n), accum="fp16")
+    assert desc["kernel"].startswith(f"ta_fwd_rowsl_n{tile_n}_"), desc
+    say(f"{desc['kernel']} {shape} {layout}")
+    out = torch.ops.tiledattention.sdpa_fwd(*args, causal, None, 128, tile_n, 1)
+    torch.cuda.synchronize()
+    check_close(as_f32(out), ref, dtype, tol=TOL[dtype], what=f"rowsl {shape} {layout}")

@@ -111,6 +111,16 @@ __device__ static inline float fast_log2(float x) { return __builtin_amdgcn_logf
 __device__ static inline float vmax(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 __device__ static inline float vmax3(float a, float b, float c) { return vmax(a, vmax(b, c)); }
 
+// vmax3 kept as one instruction: the compiler re-associates a chain of them and leaves
+// two-operand steps in it (24 instructions instead of 16 for 32 values).  The empty asm sees
+// only the result, never an operand, which may be an MFMA's, whose wait states the compiler
+// inserts for its own instructions only.
+__device__ static inline float vmax3_step(float a, float b, float c) {
+  float x = vmax3(a, b, c);
+  asm("" : "+v"(x));
+  return x;
+}
+
 // 16-byte chunk swizzle of the unpadded LDS key tiles of the eight-wave and wide kernels
 // (row = 2D bytes, 64 banks x 4 bytes):
 // * K: a b128 read pass covers 16 consecutive rows at one logical chunk;

@@ -23,6 +23,15 @@
 // halves the LDS operand reads, was not faster (12.4 -> 14.1, 24.3 -> 24.4 us), nor were eight
 // waves a workgroup in general, or a raised priority for either kind of work; without any
 // softmax arithmetic the four cases above take 10-12 % less, so loads and latency bound them.
+//
+// Input-dtype accumulation (LOWP_TN): the same workgroups with the eight-wave kernel's two key
+// slices a row, both in one wave (even and odd tiles), so results and errors are the same to the
+// merge's last bit (2-norm 1e-5): C4's D = 64 shape, fp16 404 -> 362 us, bf16 402 -> 340;
+// B16 H16 S512 fp16 41 -> 29.  VALU-bound (84 % of cycles): per tile and lane 32 FMAs, 32
+// exponentials, 32 sums, 16 maxima, 16 packs, the rounding of O (48) and its rescale (32, three
+// tiles in five).  The rescale is a branch of its own in front of one rounding: a branch with a
+// rounding on either side kept a second copy of O alive (7-13 registers spilled at D = 64, over
+// 100 at 128).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -40,10 +49,16 @@ constexpr int kRowsWaves = 4;
 constexpr int kRowsExact = 3;  // tiles with the exact running max
 
 // p.n_qblk = ceil(S / 128).
-template <int DT, int D, bool CAUSAL, bool TAIL>
+template <int DT, int D, bool CAUSAL, bool TAIL, int LOWP_TN = 0>
 __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
   static_assert(D == 64 || D == 96 || D == 128 || D == 160, "head dims 64, 96, 128 and 160");
   constexpr int NW = kRowsWaves;
+  // Input-dtype accumulation: two key slices a row, the even and the odd tiles, each with its
+  // own (m, l, O): the slices, the arithmetic and the cadence of rounding (once per TILE_N keys
+  // of a slice) of the eight-wave kernel's two wave groups.
+  constexpr bool LOWP = LOWP_TN != 0;
+  constexpr int NSL = LOWP ? 2 : 1;
+  static_assert(LOWP_TN == 0 || LOWP_TN == 64 || LOWP_TN == 128, "TILE_N");
   constexpr int TK = kRowsKeys;
   constexpr int TM = 32 * NW;
   constexpr int RB = 2 * D;              // bytes per key row
@@ -130,11 +145,15 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
 
   // ---- Q fragment: lane l holds row wq0 + l % 32, columns 16 kk + 8 (l / 32) .. + 8
   u32x4 qf[DK];
-  float m_run = kNegLarge;
-  float l_part = 0.0f;
-  f32x16 o_acc[DB];
+  float m_sl[NSL], l_sl[NSL];
+  f32x16 o_sl[NSL][DB];
 #pragma unroll
-  for (int db = 0; db < DB; ++db) o_acc[db] = f32x16{};
+  for (int i = 0; i < NSL; ++i) {
+    m_sl[i] = kNegLarge;
+    l_sl[i] = 0.0f;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) o_sl[i][db] = f32x16{};
+  }
 
   dma(kp, p.k_ss, k_rb, kvo, 0, lds_k0);
   dma(vp, p.v_ss, v_rb, vvo, 0, lds_v0);
@@ -148,7 +167,11 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
     }
   }
 
-  auto tile = [&](int t, const char* kst, const char* vst) {
+  auto tile = [&](int t, const char* kst, const char* vst, auto par_tag) {
+    constexpr int SL = LOWP ? decltype(par_tag)::value : 0;
+    float& m_run = m_sl[SL];
+    float& l_part = l_sl[SL];
+    f32x16(&o_acc)[DB] = o_sl[SL];
     const int k0 = t * TK;
     if (k0 >= wave_kv_end) return;
     f32x16 s[KB];
@@ -180,14 +203,57 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
       for (int bk = 0; bk < KB; ++bk) {
 #pragma unroll
         for (int r = 0; r < 16; r += 4) {
-          mxa = vmax3(mxa, s[bk][r], s[bk][r + 1]);
-          mxb = vmax3(mxb, s[bk][r + 2], s[bk][r + 3]);
+          mxa = vmax3_step(mxa, s[bk][r], s[bk][r + 1]);
+          mxb = vmax3_step(mxb, s[bk][r + 2], s[bk][r + 3]);
         }
       }
       float a0, a1;
       swap32(vmax(mxa, mxb), a0, a1);
       return vmax(a0, a1);
     };
+    if constexpr (LOWP) {
+      // Exact running max; P from it, packed for P.V; l from the unrounded P; the products
+      // accumulated since the last rounding rounded to the input dtype, rescaled first where
+      // a row's max moved (attn_fwd_pp.hip).
+      const float m_new = vmax(m_run, row_max());
+      const float alpha = fast_exp2((m_run - m_new) * c);
+      m_run = m_new;
+      const float mc = m_run * c;
+      float l4[4];
+#pragma unroll
+      for (int bk = 0; bk < KB; ++bk) {
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) {
+          const float p0 = fast_exp2(__builtin_fmaf(s[bk][r], c, -mc));
+          const float p1 = fast_exp2(__builtin_fmaf(s[bk][r + 1], c, -mc));
+          pk[bk][r >> 1] = DTy::pack(p0, p1);
+          const int j = (r >> 1) & 3;
+          l4[j] = bk == 0 && r < 8 ? p0 + p1 : l4[j] + (p0 + p1);
+        }
+      }
+      l_part = l_part * alpha + ((l4[0] + l4[1]) + (l4[2] + l4[3]));
+      const bool moved = __ballot(!(alpha == 1.0f)) != 0;
+      const float al = DTy::round(alpha);
+      const bool round_now = LOWP_TN == 64 || ((t >> 1) & 1);  // step t >> 1 of the slice
+      if (moved) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db) o_acc[db] *= al;
+      }
+      if (round_now) {
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+#pragma unroll
+          for (int r = 0; r < 16; r += 2) {
+            // (kept packed: fp16 would otherwise be converted value by value, four
+            // instructions a pair instead of three)
+            uint32_t w = DTy::pack(o_acc[db][r], o_acc[db][r + 1]);
+            asm("" : "+v"(w));
+            o_acc[db][r] = DTy::lo(w);
+            o_acc[db][r + 1] = DTy::hi(w);
+          }
+        }
+      }
+    }
     auto make_p = [&](float mc) {
 #pragma unroll
       for (int bk = 0; bk < KB; ++bk) {
@@ -215,31 +281,33 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
     // maxima a row, one a key half: with one (the first tile's) the error against 64 bits was up
     // to 4 % above its (bf16 S100 2.17e-3 against 2.07e-3, S512 2.30 against 2.27), with three
     // tiles it is at or below it from S = 197 on; every further tile costs 1 %.
-    if (t < kRowsExact) {
-      const float m_new = vmax(m_run, row_max());
-      if (t > 0 && __ballot(!(m_new == m_run))) {
-        const float alpha = fast_exp2((m_run - m_new) * c);
+    if constexpr (!LOWP) {
+      if (t < kRowsExact) {
+        const float m_new = vmax(m_run, row_max());
+        if (t > 0 && __ballot(!(m_new == m_run))) {
+          const float alpha = fast_exp2((m_run - m_new) * c);
 #pragma unroll
-        for (int db = 0; db < DB; ++db) o_acc[db] *= alpha;
-        l_part *= alpha;
-      }
-      m_run = m_new;
-    }
-    float l_step = make_p(m_run * c);
-    if (t >= kRowsExact && __ballot(!(l_step < kRescaleBound))) {
-      const float mx = row_max();
-      const bool need = (mx - m_run) * c > kRescaleLog2;
-      if (__ballot(need)) {
-        const float m_new = need ? mx : m_run;
-        const float alpha = fast_exp2((m_run - m_new) * c);
+          for (int db = 0; db < DB; ++db) o_acc[db] *= alpha;
+          l_part *= alpha;
+        }
         m_run = m_new;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) o_acc[db] *= alpha;
-        l_part *= alpha;
-        l_step = make_p(m_run * c);
       }
+      float l_step = make_p(m_run * c);
+      if (t >= kRowsExact && __ballot(!(l_step < kRescaleBound))) {
+        const float mx = row_max();
+        const bool need = (mx - m_run) * c > kRescaleLog2;
+        if (__ballot(need)) {
+          const float m_new = need ? mx : m_run;
+          const float alpha = fast_exp2((m_run - m_new) * c);
+          m_run = m_new;
+#pragma unroll
+          for (int db = 0; db < DB; ++db) o_acc[db] *= alpha;
+          l_part *= alpha;
+          l_step = make_p(m_run * c);
+        }
+      }
+      l_part += l_step;
     }
-    l_part += l_step;
 #pragma unroll
     for (int bk = 0; bk < KB; ++bk) {
 #pragma unroll
@@ -260,7 +328,7 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
 
   // Tile t: this wave's loads of it (issued a tile ago) have landed, then the barrier: every
   // wave's have, and every wave is done reading tile t - 1, whose stage takes tile t + 1.
-  auto step = [&](int t, char* k_cur, char* v_cur, char* k_nxt, char* v_nxt) {
+  auto step = [&](int t, char* k_cur, char* v_cur, char* k_nxt, char* v_nxt, auto par_tag) {
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -269,29 +337,46 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
       dma(kp, p.k_ss, k_rb, kvo, t + 1, k_nxt);
       dma(vp, p.v_ss, v_rb, vvo, t + 1, v_nxt);
     }
-    tile(t, k_cur, v_cur);
+    tile(t, k_cur, v_cur, par_tag);
   };
   for (int t = 0; t < n_tiles; t += 2) {
-    step(t, lds_k0, lds_v0, lds_k1, lds_v1);
-    if (t + 1 < n_tiles) step(t + 1, lds_k1, lds_v1, lds_k0, lds_v0);
+    step(t, lds_k0, lds_v0, lds_k1, lds_v1, std::integral_constant<int, 0>{});
+    if (t + 1 < n_tiles) step(t + 1, lds_k1, lds_v1, lds_k0, lds_v0, std::integral_constant<int, 1>{});
   }
 
   // ---- O = acc / l: the lane pair l, l + 32 holds halves of a row's 16-byte chunks; swapping
   // chunk g's upper half with chunk g + 1's lower half gives each lane a whole chunk.
-  float la, lb;
-  swap32(l_part, la, lb);
-  const float inv = 1.0f / (la + lb);
+  // (Input-dtype accumulation: the slices combined in fp32 and rounded to the input dtype, then
+  // rnd(acc rnd(1 / l)).)
+  f32x16(&o_acc)[DB] = o_sl[0];
+  float la, lb, a0 = 1.0f, a1 = 0.0f;
+  if constexpr (LOWP) {
+    const float m = vmax(m_sl[0], m_sl[NSL - 1]);
+    a0 = fast_exp2((m_sl[0] - m) * c);
+    a1 = fast_exp2((m_sl[NSL - 1] - m) * c);
+    swap32(l_sl[0] * a0 + l_sl[NSL - 1] * a1, la, lb);
+  } else {
+    swap32(l_sl[0], la, lb);
+  }
+  const float inv = LOWP ? DTy::round(1.0f / (la + lb)) : 1.0f / (la + lb);
+  if constexpr (LOWP) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o_acc[db][r] = DTy::round(o_acc[db][r] * a0 + o_sl[NSL - 1][db][r] * a1);
+    }
+  }
   uint16_t* orow = op + (int64_t)my_q * p.o_ss;
 #pragma unroll
   for (int db = 0; db < DB; ++db) {
 #pragma unroll
     for (int g = 0; g < 4; g += 2) {
-      uint32_t a0 = DTy::pack(o_acc[db][4 * g] * inv, o_acc[db][4 * g + 1] * inv);
-      uint32_t a1 = DTy::pack(o_acc[db][4 * g + 2] * inv, o_acc[db][4 * g + 3] * inv);
-      uint32_t b0 = DTy::pack(o_acc[db][4 * g + 4] * inv, o_acc[db][4 * g + 5] * inv);
-      uint32_t b1 = DTy::pack(o_acc[db][4 * g + 6] * inv, o_acc[db][4 * g + 7] * inv);
-      const auto x0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
-      const auto x1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
+      const uint32_t x0a = DTy::pack(o_acc[db][4 * g] * inv, o_acc[db][4 * g + 1] * inv);
+      const uint32_t x1a = DTy::pack(o_acc[db][4 * g + 2] * inv, o_acc[db][4 * g + 3] * inv);
+      const uint32_t x0b = DTy::pack(o_acc[db][4 * g + 4] * inv, o_acc[db][4 * g + 5] * inv);
+      const uint32_t x1b = DTy::pack(o_acc[db][4 * g + 6] * inv, o_acc[db][4 * g + 7] * inv);
+      const auto x0 = __builtin_amdgcn_permlane32_swap(x0a, x0b, false, false);
+      const auto x1 = __builtin_amdgcn_permlane32_swap(x1a, x1b, false, false);
       const int d = 32 * db + 8 * (g + hl);
       if ((!TAIL || my_q < S) && d < d_real)
         *(u32x4*)(orow + d) = u32x4{(uint32_t)x0[0], (uint32_t)x1[0], (uint32_t)x0[1], (uint32_t)x1[1]};
@@ -314,3 +399,16 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
   TA_ROWS_DEFINE(DTN, DT, D, 0, 1, WPS)      \
   TA_ROWS_DEFINE(DTN, DT, D, 1, 0, WPS)      \
   TA_ROWS_DEFINE(DTN, DT, D, 1, 1, WPS)
+
+// Input-dtype accumulation, tiles (128, TN): ta_fwd_rowsl_n<TN>_<dtype>_d<D>_c<causal>_t<tail>.
+#define TA_ROWSL_DEFINE(TN, DTN, DT, D, C, T, WPS)                                          \
+  extern "C" __global__ void __launch_bounds__(64 * ta::kRowsWaves)                         \
+      __attribute__((amdgpu_waves_per_eu(WPS, WPS)))                                        \
+      ta_fwd_rowsl_n##TN##_##DTN##_d##D##_c##C##_t##T(ta::FwdParams p) {                    \
+    ta::attn_fwd_rows_body<DT, D, (C != 0), (T != 0), TN>(p);                               \
+  }
+#define TA_ROWSL_DEFINE_CT(TN, DTN, DT, D, WPS)   \
+  TA_ROWSL_DEFINE(TN, DTN, DT, D, 0, 0, WPS)      \
+  TA_ROWSL_DEFINE(TN, DTN, DT, D, 0, 1, WPS)      \
+  TA_ROWSL_DEFINE(TN, DTN, DT, D, 1, 0, WPS)      \
+  TA_ROWSL_DEFINE(TN, DTN, DT, D, 1, 1, WPS)

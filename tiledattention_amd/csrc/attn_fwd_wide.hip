@@ -382,3 +382,13 @@ TA_ROWS_DEFINE_CT(bf16, 1, 64, 4)
 TA_ROWS_DEFINE_CT(bf16, 1, 96, 3)
 TA_ROWS_DEFINE_CT(bf16, 1, 128, 2)
 TA_ROWS_DEFINE_CT(bf16, 1, 160, 2)
+
+// Input-dtype accumulation: three workgroups a CU at D = 64 (two O a lane: 146 VGPRs), two at 128.
+TA_ROWSL_DEFINE_CT(64, f16, 0, 64, 3)
+TA_ROWSL_DEFINE_CT(128, f16, 0, 64, 3)
+TA_ROWSL_DEFINE_CT(64, f16, 0, 128, 2)
+TA_ROWSL_DEFINE_CT(128, f16, 0, 128, 2)
+TA_ROWSL_DEFINE_CT(64, bf16, 1, 64, 3)
+TA_ROWSL_DEFINE_CT(128, bf16, 1, 64, 3)
+TA_ROWSL_DEFINE_CT(64, bf16, 1, 128, 2)
+TA_ROWSL_DEFINE_CT(128, bf16, 1, 128, 2)

@@ -699,6 +699,27 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   return S <= 768 || (S <= 1024 && n > 4 * (int64_t)ncu) || (S <= 1536 && paired && !full);
 }
 
+// Whether input-dtype accumulation on a 128-row tile runs the small-workgroup kernel
+// (ta_fwd_rowsl_*).  The exact maximum of every tile and the rounding of O make these kernels
+// VALU-bound, and in the eight-wave kernel one wave a SIMD at a time issues VALU work, every
+// seventh cycle or so; here two or three waves a SIMD do, in no fixed phase.  More blocks than
+// CUs, and (us, eight-wave -> this, bf16 TILE_N 64 unless noted):
+// * D = 64, non-causal: any S (B1 H32 S4096 211 -> 179, fp16 210 -> 186, TILE_N 128 177 -> 163);
+//   causal up to S = 1024, 2048 from three blocks a CU (64 heads 85 -> 66; 32 heads, two, TILE_N
+//   128 43.0 -> 42.9) and 3072 from six (64 heads 155 -> 130; S4096 32 heads fp16 127 -> 130);
+// * D = 128, TILE_N 64: non-causal up to S = 4096 (16 heads 158 -> 149), causal as D = 64 to
+//   2048 (64 heads 119 -> 109, S3072 32 heads 116 -> 124); TILE_N 128, half the rounding:
+//   non-causal up to 768 (128 heads 51.0 -> 49.2, S1024 64 heads 41.4 -> 41.4), causal up to
+//   512 (128 heads 26.6 -> 23.1, S768 43.0 -> 43.7).
+bool use_rowsl(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
+  if (a->tile_m != 128 || !eight_wave_lowp(a->tile_m, a->tile_n, a->accum, a->D) || ncu <= 0) return false;
+  const int64_t S = a->S, n = n_bh * n_qblk;
+  if (n <= ncu) return false;
+  if (a->D == 128 && a->tile_n == 128) return S <= (a->causal ? 512 : 768);
+  if (!a->causal) return a->D == 64 || S <= 4096;
+  return S <= 1024 || (S <= 2048 && n >= 3 * (int64_t)ncu) || (a->D == 64 && S <= 3072 && n >= 6 * (int64_t)ncu);
+}
+
 // Whether split key ranges exist for this configuration: the eight-wave kernels with fp32
 // accumulation, 128-row blocks (chunks and the paired split) or 64-row blocks (chunks, each
 // 128-row item of the numbering run as two 64-row halves).
@@ -794,6 +815,11 @@ ta_status plan_launch(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int32_
   if (use_rows(a, n_bh, n_qblk, ncu)) {
     char name[64];
     snprintf(name, sizeof(name), "ta_fwd_rows_%s_d%d_c%d_t%d", dt, (int)a->D, a->causal ? 1 : 0, aligned ? 0 : 1);
+    pl->main = KernelId{kWideObject, name, 256u};
+  } else if (use_rowsl(a, n_bh, n_qblk, ncu)) {
+    char name[64];
+    snprintf(name, sizeof(name), "ta_fwd_rowsl_n%d_%s_d%d_c%d_t%d", (int)a->tile_n, dt, (int)a->D, a->causal ? 1 : 0,
+             aligned ? 0 : 1);
     pl->main = KernelId{kWideObject, name, 256u};
   } else if (eight_wave(a->tile_m, a->tile_n, a->accum, a->D)) {
     if (a->causal && use_pairs(a, n_bh, n_qblk, ncu)) {
@@ -1162,9 +1188,9 @@ ta_status ta_prepare(int32_t device, int32_t dtype, int32_t head_dim, int32_t ti
   }
   ta_status st = get_function_locked(
       device, kernel_id(dtype, head_dim, tile_m, tile_n, causal != 0, aligned == 0, accum), &fn);
-  if (st != TA_OK || accum != TA_ACC_FP32 || head_dim > 160) return st;
-  // Short rows run kernels of another code object (use_wide, use_rows): loaded here too, so
-  // that a launch, which may be captured, finds it (a failure is that launch's to report).
+  if (st != TA_OK || head_dim > (accum == TA_ACC_FP32 ? 160 : 128)) return st;
+  // Some launches run kernels of another code object (use_wide, use_rows, use_rowsl): loaded
+  // here too, so that one, which may be captured, finds it (a failure is its to report).
   hipModule_t mod = nullptr;
   (void)load_module_locked(device, kWideObject, &mod);
   return TA_OK;
