@@ -172,6 +172,7 @@ def describe(lib: ctypes.CDLL, args: "FwdArgs", chunk_steps: int = 0,
 
 _lock = Lock()
 _lib: ctypes.CDLL | None = None
+_call = None
 
 
 def lib_dir() -> Path:
@@ -274,6 +275,33 @@ def load() -> ctypes.CDLL:
             raise DependencyError(f"ta_set_code_object_dir failed: {last_error(lib)}")
         _lib = lib
         return lib
+
+
+def load_call():
+    """The CPython module ``_tiledattn_call`` beside the library (``launch``: a planned call's
+    allocation and launch), loaded once per process; ``DependencyError`` if absent."""
+    global _call
+    with _lock:
+        if _call is None:
+            path = lib_dir() / "_tiledattn_call.so"
+            if not path.exists():
+                raise DependencyError(
+                    f"Native call module {path} is missing. Build it with "
+                    "`python -m tiledattention_amd.csrc.build`."
+                )
+            try:
+                spec = importlib.util.spec_from_file_location("_tiledattn_call", path)
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+            except ImportError as exc:
+                raise DependencyError(f"Native call module {path} could not be loaded: {exc}") from exc
+            _call = mod
+        return _call
+
+
+def loaded_call():
+    """``_tiledattn_call`` if ``load_call()`` already succeeded in this process, else None."""
+    return _call
 
 
 def loaded() -> ctypes.CDLL | None:

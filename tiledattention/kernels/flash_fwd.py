@@ -517,10 +517,13 @@ class _LaunchPlan:
 
     __slots__ = ("generation", "empty", "out_shape", "out_like_q", "head_dim", "pad_dim", "width",
                  "copy", "args", "kernel", "chunk", "ws_bytes", "sync_mode", "device",
-                 "device_index", "dtype")
+                 "device_index", "dtype", "launch", "fn_addr", "args_addr")
 
 
 _PLANS: dict[tuple, _LaunchPlan] = {}
+# The same plans by the tensors' layout as one bytes key (_tiledattn_call.layout), which plain
+# tensors are looked up by: building the tuple key takes 0.8 us of a call, this one 0.3.
+_PLANS_BY_LAYOUT: dict[tuple, _LaunchPlan] = {}
 _PLANS_MAX = 512
 
 
@@ -674,6 +677,7 @@ def _build_plan(torch_mod, lib, q, k, v, causal: bool, tile: tuple[int, int] | N
     plan.out_like_q = width == head_dim
     plan.sync_mode = sync_mode
     plan.empty = batch * heads == 0 or seq_len == 0
+    plan.launch = None
     if plan.empty:
         return plan
 
@@ -719,19 +723,38 @@ def _build_plan(torch_mod, lib, q, k, v, causal: bool, tile: tuple[int, int] | N
     plan.chunk = pol.chunk
     plan.ws_bytes = pol.ws_bytes
     plan.args = args
+    # A call of plain tensors that launches one kernel over inputs read in place, without a
+    # sync mode, goes from its plan to the launch natively (_tiledattn_call).
+    if (type(q) is torch_mod.Tensor and plan.out_like_q and sync_mode == "async" and not plan.ws_bytes
+            and not any(plan.copy)):
+        plan.launch = _lib.load_call().launch
+        plan.fn_addr = ctypes.cast(lib.ta_sdpa_fwd, ctypes.c_void_p).value
+        plan.args_addr = ctypes.addressof(args)
     return plan
 
 
 def _plan_for(torch_mod, q, k, v, causal: bool, tile, accum) -> _LaunchPlan:
     """The cached launch plan of a call (built on the first call of a configuration)."""
-    key = (q.shape, q.stride(), k.stride(), v.stride(), q.dtype, q.device, causal, _knob_snapshot(),
-           tile, accum)
+    call = _lib.loaded_call()
+    layout = call.layout(q, k, v) if call is not None else None
+    knobs = _knob_snapshot()
+    if layout is not None:
+        fast = (layout, causal, knobs, tile, accum)
+        plan = _PLANS_BY_LAYOUT.get(fast)
+        if plan is not None and plan.generation == _compile_cache.generation():
+            return plan
+    key = (q.shape, q.stride(), k.stride(), v.stride(), q.dtype, q.device, causal, knobs, tile, accum)
     plan = _PLANS.get(key)
     if plan is None or plan.generation != _compile_cache.generation():
         plan = _build_plan(torch_mod, _runtime.get_native_library(), q, k, v, causal, tile, accum)
         if len(_PLANS) >= _PLANS_MAX:
             _PLANS.clear()
+            _PLANS_BY_LAYOUT.clear()
         _PLANS[key] = plan
+    if layout is not None:
+        if len(_PLANS_BY_LAYOUT) >= _PLANS_MAX:
+            _PLANS_BY_LAYOUT.clear()
+        _PLANS_BY_LAYOUT[fast] = plan
     return plan
 
 
@@ -767,7 +790,8 @@ def run_flash_fwd(
     padded on the host).  K is read row-major in place; no
     transposed view or per-call copy is made unless the inputs' strides require one.  The
     resolution is cached per configuration and knob values (``_build_plan``); a call then
-    allocates the output, fills the tensor addresses and scale, and launches.
+    allocates the output, fills the tensor addresses and scale, and launches, natively where
+    nothing has to be copied (``_LaunchPlan.launch``).
 
     ``tile`` (TILE_M, TILE_N) and ``accum`` ('fp32' | 'fp16'), when given, override the
     corresponding knobs (the custom operator passes its arguments this way); ``sdpa`` leaves
@@ -775,6 +799,13 @@ def run_flash_fwd(
     """
     torch_mod = _runtime.get_torch_module()
     plan = _plan_for(torch_mod, q, k, v, causal, tile, accum)
+
+    if plan.launch is not None:
+        out = plan.launch(plan.fn_addr, plan.args_addr, q, k, v, scale)
+        if type(out) is int:
+            _raise_for_status(plan.kernel.lib, out)
+        elif out is not None:
+            return out
 
     if plan.out_like_q and type(q) is torch_mod.Tensor:
         out = torch_mod.empty_like(q, memory_format=torch_mod.contiguous_format)

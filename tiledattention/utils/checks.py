@@ -14,6 +14,7 @@ from __future__ import annotations
 
 from types import ModuleType
 
+from .. import _lib
 from .._errors import DTypeNotSupportedError, InvalidShapeError
 
 
@@ -25,6 +26,9 @@ def _ensure_tensor(torch_mod: ModuleType, name: str, value: object) -> None:
 
 def validate_sdpa_inputs(torch_mod: ModuleType, q, k, v) -> None:
     """Check the SDPA input contract; raise the first violation found."""
+    call = _lib.loaded_call()
+    if call is not None and call.valid(q, k, v):  # the check below, natively
+        return
     tensor_type = torch_mod.Tensor
     if type(q) is tensor_type and type(k) is tensor_type and type(v) is tensor_type:
         # Every check below at once (plain tensors, 4-d, one shape, one CUDA device, one

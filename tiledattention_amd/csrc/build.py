@@ -13,7 +13,9 @@ Outputs (into ``tiledattention_amd/lib/`` unless told otherwise):
   ``tiledattn.cpp`` (g++) and ``tiledattn_static.hip`` (hipcc; the static device scratch of
   ``ta_sdpa_fwd_split_static``);
 * ``libtiledattn_torch.so``: the C++ torch operator ``tiledattention::sdpa_fwd``
-  (``torch_ext.cpp``, g++ against the installed torch), linked to ``libtiledattn.so``.
+  (``torch_ext.cpp``, g++ against the installed torch), linked to ``libtiledattn.so``;
+* ``_tiledattn_call.so``: the native tail of a Python call (``py_call.cpp``, a CPython
+  extension module over the installed torch).
 
 Run as ``python -m tiledattention_amd.csrc.build``.
 """
@@ -165,12 +167,53 @@ def torch_ext_cmd(out_dir: Path) -> list[str]:
     ]
 
 
+def py_call_cmd(out_dir: Path) -> list[str]:
+    """The CPython module ``_tiledattn_call`` (plan to launch), against the installed torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    tlib = Path(torch.__file__).resolve().parent / "lib"
+    abi = int(bool(getattr(torch._C, "_GLIBCXX_USE_CXX11_ABI", True)))
+    return [
+        os.environ.get("CXX", "g++"),
+        "-O2",
+        "-std=c++17",
+        "-fPIC",
+        "-shared",
+        "-Wall",
+        "-D__HIP_PLATFORM_AMD__",
+        "-DUSE_ROCM",
+        f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+        *[f"-I{p}" for p in cpp_extension.include_paths()],
+        f"-I{sysconfig.get_paths()['include']}",
+        f"-I{ROCM / 'include'}",
+        f"-I{REPO / 'include'}",
+        "-o",
+        str(out_dir / "_tiledattn_call.so"),
+        str(HERE / "py_call.cpp"),
+        f"-L{tlib}",
+        f"-Wl,-rpath,{tlib}",
+        "-ltorch_python",
+        "-ltorch",
+        "-ltorch_cpu",
+        "-lc10",
+        "-lc10_hip",
+        "-ltorch_hip",
+        f"-L{ROCM / 'lib'}",
+        f"-Wl,-rpath,{ROCM / 'lib'}",
+        "-lamdhip64",
+    ]
+
+
 def _build_library(out_dir: Path) -> None:
     with tempfile.TemporaryDirectory(prefix="tiledattn_build_") as tmp:
         obj = Path(tmp) / "tiledattn_static.o"
         _run(static_object_cmd(obj))
         _run(library_cmd(out_dir, obj))
     _run(torch_ext_cmd(out_dir))
+    _run(py_call_cmd(out_dir))
 
 
 def build(out_dir: Path | None = None, jobs: int | None = None) -> Path:
