@@ -30,7 +30,7 @@ struct FwdParams {
   int32_t split_slots; // partial slots per (b, h)
   int32_t d_real;      // head-dim columns present in q/k/v/o (eight-wave kernel; <= D,
                        // multiple of 8): columns d_real..D-1 read as zero, are not written
-  int32_t pad0;
+  int32_t head_group;  // whole_item's group: heads an XCD takes at a time (0 or 1: one by one)
   // Split launches merged in the kernel: arrival counters of this launch's split blocks
   // (counter slot0 of a block, see WorkItem), zero on entry and left zero; null when a
   // merge kernel follows instead.

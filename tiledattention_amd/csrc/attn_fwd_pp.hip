@@ -1262,7 +1262,7 @@ __device__ __forceinline__ void attn_fwd_pp_body(const FwdParams& p) {
     } else {
       wi = SPLIT ? split_item(blockIdx.x, p.n_bh, p.split_items, p.sched, CAUSAL, p.split_c, p.split_ns,
                               p.split_slots, p.S)
-                 : whole_item(blockIdx.x, p.n_bh, p.n_qblk, p.sched, CAUSAL);
+                 : whole_item(blockIdx.x, p.n_bh, p.n_qblk, p.sched, CAUSAL, CAUSAL ? p.head_group : 0);
     }
     attn_fwd_pp_block<DT, D, CAUSAL, TAIL, SPLIT, TMR, LOWP_TN>(p, wi, lds_k0, lds_k1, lds_v0, lds_v1);
     if (merge_here && wi.slot >= 0)

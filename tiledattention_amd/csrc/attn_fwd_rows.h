@@ -82,7 +82,7 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
   const int l32 = lane & 31;
   const int hl = lane >> 5;
 
-  const WorkItem wi = whole_item(blockIdx.x, p.n_bh, p.n_qblk, p.sched, CAUSAL);
+  const WorkItem wi = whole_item(blockIdx.x, p.n_bh, p.n_qblk, p.sched, CAUSAL, CAUSAL ? p.head_group : 0);
   const int S = p.S;
   const int b = wi.bh / p.H;
   const int h = wi.bh - b * p.H;

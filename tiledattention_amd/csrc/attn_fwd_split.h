@@ -132,11 +132,21 @@ struct WorkItem {
 // per CU before the next), the heavier half comes first and the lighter half follows from
 // the lightest up, so the j-th and (j + nq/2)-th blocks of a head, which share a CU, add up
 // to the same work.
-TA_HD inline WorkItem whole_item(int blk, int n_bh, int nq, int sched, bool causal) {
+// group > 1 (causal, sched 1, 8 | n_bh; FwdParams::head_group): an XCD takes its n_bh / 8 heads
+// `group` at a time, every head's heaviest block before any head's second, so that the heavy
+// blocks of the last heads do not start when the light ones of the first have ended.
+TA_HD inline WorkItem whole_item(int blk, int n_bh, int nq, int sched, bool causal, int group = 0) {
   const int total = nq * n_bh;
   WorkItem w;
   int j;
-  if (sched >= 1 && (total & 7) == 0) {
+  if (group > 1) {
+    const int hx = n_bh >> 3, x = blk & 7, k = blk >> 3;
+    const int first = k / (group * nq) * group;  // the group's first head on this XCD
+    const int heads = hx - first < group ? hx - first : group;
+    const int i = k - first * nq;
+    j = i / heads;
+    w.bh = x * hx + first + (i - j * heads);
+  } else if (sched >= 1 && (total & 7) == 0) {
     xcd_order(blk, n_bh, nq, &w.bh, &j);
   } else {
     w.bh = blk / nq;

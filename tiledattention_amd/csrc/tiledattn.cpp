@@ -750,7 +750,33 @@ struct LaunchPlan {
   int64_t merge_grid = 0;
   SplitLayout split;     // valid when merge
   int64_t ws_bytes = 0;  // split workspace
+  int32_t head_group = 0;  // FwdParams::head_group
 };
+
+// Heads an XCD takes at a time (FwdParams::head_group) in a causal whole-row grid of 128-row
+// blocks, `resident` of its workgroups on a CU; 0 keeps them one after the other.  One by one,
+// the last heads' heavy blocks start when the first heads' light ones have ended, and set the
+// time: taken together, bf16 B1 H32 S1500 D = 128 31.0 -> 26.3 us, D = 256 57.0 -> 46.5, D = 160
+// H64 S2048 102 -> 93, outputs bit-identical.  Where it does not help: two heads an XCD with
+// little more than a block a CU (H16 S2500, 40 blocks for 32 CUs: D = 64 22.9 -> 23.3), and a
+// grid resident at once whose heads have an odd number of blocks (blocks k and k + CUs share a
+// CU, which mixes heavy and light by itself: small workgroups, D = 64 96 heads S640 13.4 -> 14.1;
+// with an even number like meets like: 64 heads S1536 31.5 -> 29.6), nor small workgroups of
+// heads of two or three blocks (D = 64 192 heads S200 9.1 -> 9.7).  The heads taken together
+// keep their K and V in the XCD's 4 MiB of L2 (D = 256 64 heads S2048, 2 MiB a head: two at a
+// time 143 us, four 144, eight 150; D = 128 48 heads S1100: two 26.9, six 25.4), two to eight of
+// them, in even groups: a last head by itself starts its heavy block last (D = 256 40 heads
+// S2048 as 2 + 2 + 1 98 -> 111).
+int32_t head_group(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int resident, int ncu) {
+  if (!a->causal || a->sched != 1 || n_bh % 8 != 0 || n_bh < 16 || ncu < 8) return 0;
+  const int64_t heads = n_bh / 8, blocks = heads * n_qblk, cus = ncu / 8;
+  if (resident == 1 && (blocks <= cus || (heads == 2 && 8 * blocks < 11 * cus))) return 0;
+  if (resident > 1 && (n_qblk < 4 || (blocks <= cus * resident && n_qblk % 2 != 0))) return 0;
+  const int64_t fit = std::min<int64_t>(8, std::max<int64_t>(2, (int64_t{4} << 20) / (a->S * a->D * 4)));
+  int64_t groups = std::max<int64_t>(1, heads / fit);
+  if (2 * ((heads + groups - 1) / groups) >= 3 * fit && heads % (groups + 1) == 0) ++groups;
+  return static_cast<int32_t>((heads + groups - 1) / groups);
+}
 
 // The plan for shape-validated arguments with n_bh * n_qblk > 0, on a device of `ncu`
 // compute units.  chunk_steps = 0, or a chunk length that splits nothing, plans the
@@ -816,11 +842,13 @@ ta_status plan_launch(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int32_
     char name[64];
     snprintf(name, sizeof(name), "ta_fwd_rows_%s_d%d_c%d_t%d", dt, (int)a->D, a->causal ? 1 : 0, aligned ? 0 : 1);
     pl->main = KernelId{kWideObject, name, 256u};
+    pl->head_group = head_group(a, n_bh, n_qblk, a->D == 64 ? 4 : a->D == 96 ? 3 : 2, ncu);
   } else if (use_rowsl(a, n_bh, n_qblk, ncu)) {
     char name[64];
     snprintf(name, sizeof(name), "ta_fwd_rowsl_n%d_%s_d%d_c%d_t%d", (int)a->tile_n, dt, (int)a->D, a->causal ? 1 : 0,
              aligned ? 0 : 1);
     pl->main = KernelId{kWideObject, name, 256u};
+    pl->head_group = head_group(a, n_bh, n_qblk, a->D == 64 ? 3 : 2, ncu);
   } else if (eight_wave(a->tile_m, a->tile_n, a->accum, a->D)) {
     if (a->causal && use_pairs(a, n_bh, n_qblk, ncu)) {
       pl->main = pair_kernel_id(a->dtype, (int)a->D, !aligned);
@@ -836,10 +864,13 @@ ta_status plan_launch(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int32_
       pl->rows = 256;
       pl->tail = t256;
       pl->layout = TA_LAYOUT_ROWS256;
+    } else {
+      pl->head_group = head_group(a, n_bh, n_qblk, 1, ncu);
     }
   } else if (use_pp_d256(a, n_bh, n_qblk)) {
     // (tile_m divides the aligned variant's S, so its 64-key steps are whole.)
     pl->main = pp_d256_kernel_id(a->dtype, a->causal, !aligned);
+    pl->head_group = head_group(a, n_bh, n_qblk, 1, ncu);
   } else if (eight_wave64(a->tile_m, a->tile_n, a->accum, a->D) && use_wide(a->S, n_bh, a->D, ncu)) {
     // The aligned variant's S (a multiple of 128) is whole 32-row blocks and whole passes of
     // a wave's keys, as its t0 form needs.
@@ -963,6 +994,7 @@ ta_status launch_plan_locked(const ta_fwd_args* a, const ResolvedPlan& r, ta::Fw
   if (pl.layout == TA_LAYOUT_WIDE) p->n_qblk = static_cast<int32_t>((a->S + 31) / 32);
   // the split numbering and the merge count 128-row blocks, whatever rows a workgroup takes
   if (pl.merge) p->n_qblk = static_cast<int32_t>((a->S + kSplitRows - 1) / kSplitRows);
+  p->head_group = pl.head_group;
   p->merge_cnt = nullptr;
   if (pl.merge && pl.merge_in_kernel) p->merge_cnt = merge_counters_locked(a->device, stream);
   void* params[] = {p};
