@@ -340,13 +340,19 @@ def test_policy_defaults_run_the_described_kernels(lib):
     (96, False, 8, 1024, True), (96, False, 8, 1025, False),
     (128, False, 9, 512, True), (128, False, 9, 513, False),
     (160, False, 8, 768, True), (160, False, 8, 769, False),
-    (64, True, 16, 384, True), (64, True, 16, 512, False),          # 256 pairs: one full round
-    (64, True, 24, 512, True), (64, True, 8, 768, True), (64, True, 8, 1024, False),
-    (64, True, 12, 1024, True), (64, True, 32, 1024, True),         # 384 pairs; 2048 blocks
-    (96, True, 8, 1536, True), (96, True, 8, 1537, False), (96, True, 16, 1536, False),
-    (128, True, 12, 512, True), (128, True, 16, 512, False), (128, True, 8, 640, False),
-    (128, True, 16, 640, True), (128, True, 12, 768, True), (128, True, 32, 768, False),
-    (128, True, 12, 769, False), (160, True, 8, 640, True), (160, True, 8, 641, False),
+    # causal: whole heads on every XCD
+    (64, True, 16, 384, True), (64, True, 16, 512, True),
+    (64, True, 7, 1024, False), (64, True, 8, 1024, True),          # 448 / 512 blocks
+    (64, True, 6, 1280, False), (64, True, 8, 1280, True), (64, True, 8, 1536, True),
+    (64, True, 10, 1408, False), (64, True, 16, 1408, True),        # resident at once, odd; past it
+    (64, True, 6, 2048, False), (64, True, 8, 2048, True), (64, True, 10, 3073, False),
+    (96, True, 7, 896, False), (96, True, 8, 960, True), (96, True, 8, 1024, False),
+    (96, True, 8, 1536, True), (96, True, 8, 1920, True), (96, True, 8, 1921, False),
+    (128, True, 10, 388, True), (128, True, 12, 512, False), (128, True, 16, 512, False),
+    (128, True, 14, 640, True), (128, True, 9, 1024, True), (128, True, 9, 1025, False),
+    (160, True, 9, 512, True), (160, True, 8, 640, False), (160, True, 10, 640, True),
+    (160, True, 8, 1024, False), (160, True, 9, 1024, True), (160, True, 8, 1536, True),
+    (160, True, 8, 1537, False),
 ])
 def test_small_workgroup_rule(lib, objects, d, causal, b, s, rows):
     for aligned in (0, 1):
@@ -364,6 +370,21 @@ def test_small_workgroup_rule(lib, objects, d, causal, b, s, rows):
         args = dict(B=b, H=8, S=s, D=d, causal=causal, tile_m=128, sched=1)
         args.update(kw)
         assert not _d(lib, **args).kernel.decode().startswith("ta_fwd_rows_")
+
+
+# Heads that the XCDs cannot take whole: small workgroups and pairs by the grid's size alone.
+@pytest.mark.parametrize("d,h,s,family", [
+    (64, 129, 512, "rows"), (64, 63, 1024, "pp"), (64, 65, 1024, "rows"), (64, 129, 1024, "rows"), (64, 129, 1537, "pp_pair"),
+    (128, 129, 512, "rows"), (128, 65, 640, "pp"), (128, 129, 640, "rows"), (128, 129, 769, "pp_pair"),
+    (160, 65, 640, "rows"), (160, 65, 641, "pp"),
+    # whole heads on every XCD: pairs only where they fill the rounds of the CUs
+    (128, 32, 2048, "pp_pair"), (128, 40, 2048, "pp"), (128, 41, 2048, "pp_pair"), (128, 40, 3072, "pp_pair"),
+    (128, 40, 3200, "pp_pair"), (128, 48, 2688, "pp"),  # eight single blocks left over; sixteen of 24
+])
+def test_causal_family(lib, objects, d, h, s, family):
+    desc = _d(lib, B=1, H=h, S=s, D=d, causal=True, tile_m=128, sched=1)
+    assert desc.kernel.decode() == f"ta_fwd_{family}_bf16_d{d}_c1_t{int(s % 128 != 0)}"
+    assert desc.kernel + b"\x00" in objects[desc.code_object.decode()]
 
 
 # The same workgroups with input-dtype accumulation: 128-row tiles, more blocks than CUs.

@@ -609,11 +609,24 @@ bool unmasked_tail(const ta_fwd_args* a) {
   return a->aligned == 1 && a->S % a->tile_m == 0 && a->S % a->tile_n == 0 && steps;
 }
 
+// Whether the causal pairs of a grid fill its rounds of the CUs: 85 % or more of them, or all but a
+// last one of a fiftieth of the pairs that is the heads' middle blocks by themselves (odd n_qblk:
+// bf16 D = 128 40 heads S3200, 520 pairs, whole blocks 1.06 of the pairs' time).
+bool pairs_fill(int64_t n_bh, int64_t n_qblk, int ncu) {
+  const int64_t pairs = n_bh * ((n_qblk + 1) / 2), rounds = (pairs + ncu - 1) / ncu;
+  const int64_t last = pairs - (rounds - 1) * ncu;
+  return 100 * pairs >= 85 * rounds * ncu || (rounds > 1 && n_qblk % 2 != 0 && 50 * last <= pairs);
+}
+
 // Whether a whole-row launch runs causal query blocks in pairs (nq - 1 - j, then j; one
 // workgroup each pair, attn_fwd_split.h pair_items): the eight-wave kernel at D <= 128,
 // causal, at least two blocks a head, and either forced (sched 3) or, with XCD grouping
 // (sched 1), a grid of two or more workgroups per CU.  Below that every block runs at once and pairing would
-// only lengthen the longest workgroup.  With two waves of workgroups or more, the hardware
+// only lengthen the longest workgroup.  Where every XCD has whole heads, pairs that do not
+// fill the rounds of the CUs (pairs_fill) lose to whole blocks, heaviest first over the heads
+// (head_group): bf16 D = 128 H40 S2048, 320 pairs, 62.5 -> 49.2 us, 384 pairs
+// (H48 S2048) 63.1 -> 56.8, 640 (H64 S2500) 117 -> 109; at 94 % (H40 S3072, 480) 93.8 -> 95.6.
+// With two waves of workgroups or more, the hardware
 // hands block ids to the XCDs in a fixed round-robin, so an XCD whose CUs finish early
 // waits for the others before it gets its next block; pairs give every workgroup the same
 // work (nq + 1 key steps) instead of relying on that order.
@@ -622,7 +635,8 @@ bool use_pairs(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (!a->causal || n_qblk < 2 || a->D > 128 || !eight_wave(a->tile_m, a->tile_n, a->accum, a->D))
     return false;
   if (a->sched == 3) return true;
-  return a->sched == 1 && n_bh * n_qblk >= 2 * (int64_t)ncu;
+  if (a->sched != 1 || n_bh * n_qblk < 2 * (int64_t)ncu) return false;
+  return n_bh % 8 != 0 || pairs_fill(n_bh, n_qblk, ncu);
 }
 
 // Whether a whole-row launch runs 256-row blocks (ta_fwd_pp256_*: the two wave groups own
@@ -672,15 +686,26 @@ KernelId pp_d256_kernel_id(int dtype, int causal, int tail) {
 //   blocks (256 heads 51.3 -> 44.3; S640 64 heads 22.6 -> 23.3); D = 96 up to 1024 (64 heads
 //   32.5 -> 32.2; S1536 32 heads 36.8 -> 38.4); D = 160 up to 768 (34.0 -> 32.8; S1024 96 heads
 //   69.7 -> 70.6);
-// * causal, against pairs of blocks (two or more blocks a CU): where the pairs fill one round
-//   of the CUs (85 % or more) only up to S = 384 (D = 64 S512 128 heads 12.8 -> 13.2, D = 128
-//   20.7 -> 21.7; S384 22.6 -> 19 and more); otherwise D = 64 and 96 up to S = 768 (D = 64 S512
-//   192 heads 25.3 -> 18.5), to 1024 past four blocks a CU (256 heads 66.6 -> 57), and to 1536
-//   where the pairs' last round is short (S1536 64 heads, 384 pairs, 38.0 -> 32.4, 512 pairs
-//   S1024 33.6 -> 34.3); D = 128 up to 512, 640 past two blocks a CU (S640 192 heads 48.5 ->
-//   40.0, 64 heads 18.3 -> 20.1) and 768 where the pairs' last round is short (192 heads 61.9
-//   -> 52, 256 heads 65.1 -> 65.6); D = 160, which has no pairs, up to 640 (96 heads 28.4 ->
-//   24.8; S768 35.3 -> 37.1).
+// * causal, whole heads on every XCD (8 | B H; both kernels then order a grid's heads together,
+//   head_group).  Against the faster of pairs and whole blocks, per length S and blocks n:
+//   D = 64 up to S = 768, 1024 from two blocks a CU (112 heads 0.69-0.76 of the time; 40 heads
+//   S896 11.6 -> 14.4 us), 1536 from 2.25 (64 heads 30.5 -> 26.9) and 3072 from 3.75 (S2048 64
+//   heads 46.3 -> 42.3; 48 heads S1800 34.9 -> 37.4, 64 heads S4096 153 -> 157), but not a
+//   grid past S = 1280 that is resident at once, ungrouped (odd n_qblk) and whose pairs fill
+//   their last round (80 heads S1408: 1.07 of the time);
+//   D = 96 up to 768, 960 from two blocks a CU (64 heads 0.91; 56 heads S896 1.08), 1536 from
+//   2.25 (S1024 48 heads 19.4 -> 20.3) and 1920 from 3.75 (S1800 64 heads 56.8 -> 48.9, S2048
+//   60.0 -> 63.7);
+//   D = 128 up to 384, 448 below 1.5 blocks a CU (80 heads S388 15.6 -> 13.0) and 1024 past two
+//   (112 heads S540 27.1 -> 20.6, 96 heads S640 19.2 -> 20.9, 48 heads S1536 37.3 -> 38.6);
+//   D = 160, which has no pairs, up to 512, 768 from 1.5 blocks a CU (96 heads 34.6 -> 30.7,
+//   64 heads S640 20.6 -> 22.6), 1024 from 2.25 (96 heads 46.3 -> 41.2, 48 heads 26.0 -> 28.3)
+//   and 1536 from three (64 heads 58.1 -> 55.2; 80 heads S1792 1.08 of the time);
+// * causal otherwise: where the pairs of a grid of two blocks a CU or more fill one round of
+//   the CUs only up to S = 384 (D = 64 S512 128 heads 12.8 -> 13.2); else D = 64 and 96 up to
+//   768, 1024 past four blocks a CU, and 1536 where the pairs' last round is short; D = 128 up
+//   to 512, 640 past two blocks a CU (S640 64 heads 18.3 -> 20.1) and 768 where the pairs' last
+//   round is short; D = 160 up to 640.
 bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (!eight_wave(a->tile_m, a->tile_n, a->accum, a->D) || a->sched == 3 || ncu <= 0) return false;
   const int64_t S = a->S, n = n_bh * n_qblk;
@@ -689,12 +714,20 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
     if (a->D == 64) return S <= 512 || (S <= 1024 && n >= 4 * (int64_t)ncu);
     return S <= (a->D == 96 ? 1024 : a->D == 128 ? 512 : 768);
   }
+  if (S <= 384) return true;
+  if (n_bh % 8 == 0 && a->sched == 1) {
+    const int64_t cu = ncu;
+    const bool n225 = 4 * n >= 9 * cu, n375 = 4 * n >= 15 * cu;
+    if (a->D == 160) return S <= 512 || (S <= 768 && 2 * n >= 3 * cu) || (S <= 1024 && n225) || (S <= 1536 && n >= 3 * cu);
+    if (a->D == 128) return (S <= 448 && 2 * n <= 3 * cu) || (S <= 1024 && n > 2 * cu);
+    if (a->D == 96) return S <= 768 || (S <= 960 && n >= 2 * cu) || (S <= 1536 && n225) || (S <= 1920 && n375);
+    if (S <= 1280) return S <= 768 || (S <= 1024 && n >= 2 * cu) || n225;
+    return (n_qblk % 2 == 0 || n > 4 * cu || !pairs_fill(n_bh, n_qblk, ncu)) && ((S <= 1536 && n225) || (S <= 3072 && n375));
+  }
   if (a->D == 160) return S <= 640;
   const bool paired = n >= 2 * (int64_t)ncu;
-  const int64_t pairs = n_bh * ((n_qblk + 1) / 2), rounds = (pairs + ncu - 1) / ncu;
-  const bool full = 100 * pairs >= 85 * rounds * ncu;  // the pairs' last round
-  if (S <= 384) return true;
-  if (paired && full && rounds == 1) return false;
+  const bool full = pairs_fill(n_bh, n_qblk, ncu);
+  if (paired && full && n_bh * ((n_qblk + 1) / 2) <= ncu) return false;
   if (a->D == 128) return S <= 512 || (S <= 640 && paired) || (S <= 768 && paired && !full);
   return S <= 768 || (S <= 1024 && n > 4 * (int64_t)ncu) || (S <= 1536 && paired && !full);
 }
