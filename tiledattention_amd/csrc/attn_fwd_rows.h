@@ -23,6 +23,10 @@
 // halves the LDS operand reads, was not faster (12.4 -> 14.1, 24.3 -> 24.4 us), nor were eight
 // waves a workgroup in general, or a raised priority for either kind of work; without any
 // softmax arithmetic the four cases above take 10-12 % less, so loads and latency bound them.
+// A second copy of the tile for a last one of at most 32 keys (bit-identical) was faster where such
+// rows are short (B64 H12 S80 D64 9.5 -> 8.9 us, B32 H12 S197 14.2 -> 13.7), but the copy itself costs
+// every other row 2-4 % (S250 14.7 -> 15.3, D96 S1000 58.3 -> 60.6, causal D64 S512 21.7 -> 22.2) and
+// the input-dtype kernels spill with it.
 //
 // Input-dtype accumulation (LOWP_TN): the same workgroups with the eight-wave kernel's two key
 // slices a row, both in one wave (even and odd tiles), so results and errors are the same to the
