@@ -219,7 +219,8 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
   // RPC g + l / CPR, so it loads logical chunk (l % CPR) ^ swz(row) of that row.  Rows
   // RPC NW i apart: K's swizzle repeats every 16 rows (KP distinct per-lane offsets, the
   // rest a uniform row step), V's every 4 (one offset).  Rows past S are outside the
-  // tile's buffer resource and read as zero.
+  // tile's buffer resource and read as zero; the row steps go into the per-lane offset, as a
+  // load's scalar offset is no part of its documented range check.
   constexpr int RPC = 1024 / (2 * D);
   constexpr int NCH = TN * 2 * D / 1024;
   constexpr int NLW = NCH / NW;  // loads per wave per tensor per tile
@@ -249,7 +250,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
     for (int i = 0; i < NLW; ++i) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           kr, (__attribute__((address_space(3))) void*)(base + (wave + NW * i) * 1024), 16,
-          dm_k[i % KP], (i / KP) * 16 * k_rb, 0, 0);
+          dm_k[i % KP] + (i / KP) * 16 * k_rb, 0, 0, 0);
     }
   };
   auto dma_v = [&](int kt, int stage) {
@@ -259,7 +260,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
     for (int i = 0; i < NLW; ++i) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           vr, (__attribute__((address_space(3))) void*)(base + (wave + NW * i) * 1024), 16,
-          dm_v, i * RSTEP * v_rb, 0, 0);
+          dm_v + i * RSTEP * v_rb, 0, 0, 0);
     }
   };
 

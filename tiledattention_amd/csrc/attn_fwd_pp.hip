@@ -252,9 +252,8 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   const int q_rb = (int)p.q_ss * 2;
   const int qvo = 8 * lck < d_real ? ld_row * q_rb + (lck << 4) : kZeroChunk;
   const int tqvo = DA + 8 * tl_lck < d_real ? tl_row * q_rb + 2 * DA + (tl_lck << 4) : kZeroChunk;
-  // A chunk's row step from the wave's first goes into the per-lane offset, or at D = 256,
-  // where registers are short, into the load's scalar offset (which the range check includes).
-  constexpr bool kScalarStep = D == 256;
+  // A chunk's row step from the wave's first goes into the per-lane offset: a load's scalar
+  // offset is no part of its documented range check, which zeroes rows past S.
   constexpr int KCH = pp_k_chunk(D);
   auto dma = [&](const uint16_t* gbase, int64_t row_stride, int rb, int vo, int tvo, int t, char* stage,
                  int chunk_bytes) {
@@ -265,7 +264,7 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
     for (int i = 0; i < NLD; ++i) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           r, (__attribute__((address_space(3))) void*)(stage + (ld_g0 + LS * i) * chunk_bytes), 16,
-          kScalarStep ? vo : vo + i * LS * RPL * rb, kScalarStep ? i * LS * RPL * rb : 0, 0, 0);
+          vo + i * LS * RPL * rb, 0, 0, 0);
     }
     if constexpr (NLDT != 0) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
