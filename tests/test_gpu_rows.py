@@ -8,7 +8,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from tests.parity_util import TOL, as_f32, check_close, inputs, oracle_f32, say
+from tests.parity_util import TOL, as_f32, check_close, inputs, knobs, oracle_f32, say
 
 pytestmark = pytest.mark.gpu
 
@@ -73,6 +73,62 @@ def test_rows_rescale_between_tiles(gpu, d):
     # nearly one-hot rows: P's rounding (u = 2^-8) moves O by up to 3 u max|v|
     tol = 3 * 2.0 ** -8 * float(v.float().abs().max())
     check_close(_run((q, k, v), False), ref, "bfloat16", tol=tol, what=f"rows rescale D={d}")
+
+
+def _error_against_64_bits(args, causal):
+    """(rows kernel, eight-wave kernel): 2-norm of the error over 2-norm of the exact result."""
+    import torch
+
+    from tiledattention import sdpa
+    from tiledattention.kernels import flash_fwd
+
+    q, k, v = (t.flatten(0, 1).double() for t in args)
+    kt = k.transpose(1, 2).contiguous()
+    scores = torch.matmul(q * q.shape[-1] ** -0.5, kt)
+    if causal:
+        scores.masked_fill_(torch.ones_like(scores[0], dtype=torch.bool).triu(1), float("-inf"))
+    exact = torch.matmul(torch.softmax(scores, dim=-1), v)
+    errors = []
+    for sched, family in ((None, "ta_fwd_rows_"), (3, "ta_fwd_pp_")):  # order 3 keeps the eight-wave kernel
+        with knobs(sched=sched):
+            assert flash_fwd.describe_call(*args, causal=causal)["kernel"].startswith(family)
+            out = sdpa(*args, causal=causal).flatten(0, 1).double()
+        errors.append(float((out - exact).norm() / exact.norm()))
+    return errors
+
+
+@pytest.mark.parametrize("shape,causal,dtype", [
+    ((40, 8, 70, 64), False, "float16"),
+    ((40, 8, 96, 128), False, "bfloat16"),
+    ((40, 8, 113, 160), False, "float16"),
+    ((40, 8, 128, 64), False, "bfloat16"),
+    ((40, 8, 131, 96), False, "bfloat16"),
+    ((40, 8, 128, 96), True, "float16"),
+    ((40, 8, 150, 64), True, "bfloat16"),
+    ((40, 8, 192, 128), True, "float16"),
+    ((40, 8, 256, 64), False, "float16"),
+])
+def test_rows_error_no_larger_than_the_eight_wave_kernels(gpu, shape, causal, dtype):
+    """Rows of one to four key tiles.  Rounding P dominates the error; over more than 10^6
+    outputs the ratio of two such errors scatters by about 10^-3 (1 / sqrt of their number)."""
+    args = _on_gpu(inputs(shape, dtype, 1700 + shape[2]), "bhsd")
+    say(f"rows error against 64 bits {shape} causal={causal} {dtype}")
+    rows, eight = _error_against_64_bits(args, causal)
+    print(f"[check] rows {rows:.4e} eight-wave {eight:.4e} ratio {rows / eight:.4f}", flush=True)
+    assert rows <= 1.001 * eight
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_rows_falling_maxima(gpu, dtype):
+    """Keys that shrink tile by tile: every tile's max lies far below the one before."""
+    import torch
+
+    q, k, v = inputs((33, 8, 256, 64), dtype, 83)
+    k = (k.float() * torch.tensor([8.0, 2.0, 0.25, 0.0])[torch.arange(256) // 64][None, None, :, None]).to(k.dtype)
+    ref = oracle_f32(q, k, v, causal=True)
+    # nearly one-hot rows, as above: P's rounding u moves O by up to 3 u max|v|
+    u = 2.0 ** -8 if dtype == "bfloat16" else 2.0 ** -11
+    check_close(_run((q, k, v), True), ref, dtype, tol=3 * u * float(v.float().abs().max()), what="rows falling maxima")
 
 
 @pytest.mark.parametrize("value", [float("nan"), float("-inf")])

@@ -50,7 +50,9 @@ namespace ta {
 
 constexpr int kRowsKeys = 64;  // keys per tile
 constexpr int kRowsWaves = 4;
-constexpr int kRowsExact = 3;  // tiles with the exact running max
+constexpr int kRowsExact = 3;  // tiles with an exact max of their own
+constexpr float kRowsDrop = 7.0f;  // two drops stay below the lazy rule's 2^15
+static_assert((kRowsExact - 1) * kRowsDrop <= kRescaleLog2, "growth of O and l");
 
 // p.n_qblk = ceil(S / 128).
 template <int DT, int D, bool CAUSAL, bool TAIL, int LOWP_TN = 0>
@@ -98,6 +100,7 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
   const int v_rb = (int)p.v_ss * 2;
   const int d_real = p.d_real;
   const float c = p.scale_log2;
+  const float drop = kRowsDrop * __builtin_amdgcn_rcpf(c);  // in raw score units
 
   const int q0 = wi.qt * TM;
   const int wq0 = q0 + 32 * wave;
@@ -278,16 +281,18 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
       }
       return (l4[0] + l4[1]) + (l4[2] + l4[3]);
     };
-    // Reference point of P: the exact running max over the first kRowsExact tiles (O and l are
-    // zero at the first: nothing to rescale), so that a row's largest P there are exactly 1 and
-    // carry no rounding; from then on the lazy rule of the eight-wave kernel (the max is reduced
-    // only where some lane's sum of P reaches the bound).  The eight-wave kernel has two exact
-    // maxima a row, one a key half: with one (the first tile's) the error against 64 bits was up
-    // to 4 % above its (bf16 S100 2.17e-3 against 2.07e-3, S512 2.30 against 2.27), with three
-    // tiles it is at or below it from S = 197 on; every further tile costs 1 %.
+    // Reference point of P: over the first kRowsExact tiles each tile's own exact max (O and l
+    // are zero at the first: nothing to rescale), so that a row's largest P of every such tile is
+    // exactly 1 and carries no rounding, as in the eight-wave kernel, whose two key halves have a
+    // max each; from then on the lazy rule of that kernel (the max is reduced only where some
+    // lane's sum of P reaches the bound).  A tile whose max lies more than kRowsDrop (log2 units)
+    // below the point so far takes that much less instead, which bounds how far O and l grow.
+    // Against 64 bits, the eight-wave kernel's error = 1 (B H 264-384, N(0, 1), both dtypes):
+    // with the running max instead S96 to S113 1.014-1.016, S128 1.013, causal to S200
+    // 1.002-1.003; every further exact tile costs 1 % of the time.
     if constexpr (!LOWP) {
       if (t < kRowsExact) {
-        const float m_new = vmax(m_run, row_max());
+        const float m_new = vmax(m_run - drop, row_max());
         if (t > 0 && __ballot(!(m_new == m_run))) {
           const float alpha = fast_exp2((m_run - m_new) * c);
 #pragma unroll
