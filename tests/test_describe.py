@@ -404,3 +404,20 @@ def test_small_workgroup_rule_input_dtype(lib, objects, d, tn, causal, b, s, row
     assert (desc.grid, desc.block, desc.rows) == (8 * b * -(-s // 128), 256 if rows else 512, 128)
     d64 = _d(lib, B=b, H=8, S=s, D=d, causal=causal, tile_m=64, tile_n=tn, sched=1, accum=_lib.TA_ACC_INPUT)
     assert d64.kernel.decode().startswith("ta_fwd_ppl64_")
+
+
+# Just above one block per CU a causal grid of longer rows keeps the eight-wave kernel.
+@pytest.mark.parametrize("d,tn,h,s,rows", [
+    (64, 64, 65, 512, True), (64, 64, 52, 640, False), (64, 128, 64, 640, True),
+    (64, 64, 47, 768, False), (64, 64, 48, 768, True), (64, 128, 40, 896, False), (64, 64, 48, 896, False),
+    (64, 64, 49, 896, True), (64, 128, 35, 1024, False), (64, 64, 36, 1024, True),
+    (128, 64, 65, 512, True), (128, 64, 56, 640, False), (128, 64, 64, 640, True), (128, 64, 53, 768, False),
+    (128, 64, 40, 834, False), (128, 64, 48, 896, False), (128, 64, 49, 896, True),
+    (128, 64, 39, 1024, False), (128, 64, 40, 1024, True),
+])
+def test_small_workgroup_rule_input_dtype_near_one_block_a_cu(lib, d, tn, h, s, rows):
+    desc = _d(lib, B=1, H=h, S=s, D=d, causal=True, tile_m=128, tile_n=tn, sched=1, accum=_lib.TA_ACC_INPUT)
+    fam = "rowsl" if rows else "ppl"
+    assert desc.kernel.decode() == f"ta_fwd_{fam}_n{tn}_bf16_d{d}_c1_t{int(s % 128 != 0)}"
+    free = _d(lib, B=1, H=h, S=s, D=d, causal=False, tile_m=128, tile_n=tn, sched=1, accum=_lib.TA_ACC_INPUT)
+    assert free.kernel.decode().startswith(f"ta_fwd_rowsl_n{tn}_")  # not causal: every block is as long

@@ -738,8 +738,15 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
 // seventh cycle or so; here two or three waves a SIMD do, in no fixed phase.  More blocks than
 // CUs, and (us, eight-wave -> this, bf16 TILE_N 64 unless noted):
 // * D = 64, non-causal: any S (B1 H32 S4096 211 -> 179, fp16 210 -> 186, TILE_N 128 177 -> 163);
-//   causal up to S = 1024, 2048 from three blocks a CU (64 heads 85 -> 66; 32 heads, two, TILE_N
-//   128 43.0 -> 42.9) and 3072 from six (64 heads 155 -> 130; S4096 32 heads fp16 127 -> 130);
+//   causal up to S = 512, 1024 as below, 2048 from three blocks a CU (64 heads 85 -> 66; 32 heads,
+//   two, TILE_N 128 43.0 -> 42.9) and 3072 from six (64 heads 155 -> 130; S4096 32 heads fp16
+//   127 -> 130);
+// * causal, S = 513 to 1024: not just above one block a CU, where most CUs hold a single small
+//   workgroup, half as fast as an eight-wave one: from 9/8 blocks a CU at D = 64 (TILE_N 128, 35
+//   heads S1024 22.6 -> 23.1; 48 heads S768 0.86 of the time), 5/4 at D = 128 (fp16 56 heads S640
+//   18.9 -> 21.1, 33 heads S1024 34.7 -> 37.5; 64 heads S640 0.98, 40 heads S1024 0.79), and past
+//   4/3 for heads of seven blocks (D = 128 40 heads S834 21.5 -> 25.0, 48 heads S896 27.7 -> 30.8,
+//   D = 64 TILE_N 128 40 heads S896 13.7 -> 15.6; 55 heads 0.92 and 0.86);
 // * D = 128, TILE_N 64: non-causal up to S = 4096 (16 heads 158 -> 149), causal as D = 64 to
 //   2048 (64 heads 119 -> 109, S3072 32 heads 116 -> 124); TILE_N 128, half the rounding:
 //   non-causal up to 768 (128 heads 51.0 -> 49.2, S1024 64 heads 41.4 -> 41.4), causal up to
@@ -750,7 +757,10 @@ bool use_rowsl(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (n <= ncu) return false;
   if (a->D == 128 && a->tile_n == 128) return S <= (a->causal ? 512 : 768);
   if (!a->causal) return a->D == 64 || S <= 4096;
-  return S <= 1024 || (S <= 2048 && n >= 3 * (int64_t)ncu) || (a->D == 64 && S <= 3072 && n >= 6 * (int64_t)ncu);
+  const int64_t cu = ncu;
+  if (S <= 512) return true;
+  if (S <= 1024) return n_qblk == 7 ? 3 * n > 4 * cu : a->D == 64 ? 8 * n >= 9 * cu : 4 * n >= 5 * cu;
+  return (S <= 2048 && n >= 3 * cu) || (a->D == 64 && S <= 3072 && n >= 6 * cu);
 }
 
 // Whether split key ranges exist for this configuration: the eight-wave kernels with fp32
