@@ -421,3 +421,21 @@ def test_small_workgroup_rule_input_dtype_near_one_block_a_cu(lib, d, tn, h, s, 
     assert desc.kernel.decode() == f"ta_fwd_{fam}_n{tn}_bf16_d{d}_c1_t{int(s % 128 != 0)}"
     free = _d(lib, B=1, H=h, S=s, D=d, causal=False, tile_m=128, tile_n=tn, sched=1, accum=_lib.TA_ACC_INPUT)
     assert free.kernel.decode().startswith(f"ta_fwd_rowsl_n{tn}_")  # not causal: every block is as long
+
+
+# Where the small workgroups' grid is no multiple of 8 blocks (no XCD order) or just past a round
+# of pairs, the eight-wave kernels keep it.
+@pytest.mark.parametrize("d,causal,h,s,rows", [
+    (64, False, 65, 512, False), (64, False, 66, 512, True), (64, False, 89, 449, False), (64, False, 102, 512, True),
+    (64, False, 129, 512, True), (64, False, 179, 256, True), (64, False, 253, 256, False), (64, False, 89, 384, True),
+    (128, False, 65, 512, False), (128, False, 102, 512, True), (128, False, 179, 199, False),
+    (128, False, 160, 199, True), (128, False, 179, 192, True), (128, False, 100, 330, True), (128, False, 257, 256, True),
+    (64, True, 58, 1152, False), (64, True, 71, 1152, True), (64, True, 58, 1024, False), (96, True, 58, 1152, False),
+    (96, True, 71, 1152, True), (96, True, 53, 1536, True), (96, True, 67, 1536, False), (64, True, 67, 1536, True),
+    (128, True, 105, 576, True), (128, True, 105, 640, False), (128, True, 105, 609, False), (128, True, 107, 711, True),
+    (128, True, 107, 736, True), (128, True, 107, 768, False),
+    (160, True, 52, 640, False), (160, True, 58, 640, True), (160, True, 65, 512, True),
+])
+def test_small_workgroup_rule_without_xcd_order(lib, d, causal, h, s, rows):
+    desc = _d(lib, B=1, H=h, S=s, D=d, causal=causal, tile_m=128, sched=1)
+    assert desc.kernel.decode().startswith("ta_fwd_rows_") is rows, desc.kernel

@@ -702,15 +702,28 @@ KernelId pp_d256_kernel_id(int dtype, int causal, int tail) {
 //   64 heads S640 20.6 -> 22.6), 1024 from 2.25 (96 heads 46.3 -> 41.2, 48 heads 26.0 -> 28.3)
 //   and 1536 from three (64 heads 58.1 -> 55.2; 80 heads S1792 1.08 of the time);
 // * causal otherwise: where the pairs of a grid of two blocks a CU or more fill one round of
-//   the CUs only up to S = 384 (D = 64 S512 128 heads 12.8 -> 13.2); else D = 64 and 96 up to
-//   768, 1024 past four blocks a CU, and 1536 where the pairs' last round is short; D = 128 up
-//   to 512, 640 past two blocks a CU (S640 64 heads 18.3 -> 20.1) and 768 where the pairs' last
-//   round is short; D = 160 up to 640.
+//   the CUs only up to S = 384 (D = 64 S512 128 heads 12.8 -> 13.2); else
+//   D = 64 and 96 up to 768, 1024 past four blocks a CU, and where the pairs' last round is short
+//   1536, past 1024 from 2.25 blocks a CU (58 heads S1152 D64 25.4 -> 26.3, D96 32.2 -> 34.2; 71
+//   heads 0.94 of the time), at D = 96 up to three (67 heads S1536 52.0 -> 56.1, 53 heads 0.94);
+//   D = 128 up to 512, past two blocks a CU 640 and, where the pairs' last round is short, 768, both
+//   only with 32 rows or more missing from the last block, which the small workgroups skip (107
+//   heads S711 0.96, S768 36.2 -> 37.1; 110 heads S640 29.5 -> 30.6), or up to 640 from 2.5 blocks;
+//   D = 160 up to 512, 640 from 9/8 blocks a CU (52 heads 23.3 -> 24.2);
+// * non-causal grids that the XCDs cannot share evenly (n not a multiple of 8: both kernels then
+//   take heads in plain order, which costs the small workgroups more), one round of 256-row blocks
+//   whose rows are more than three quarters real: those at D = 128 (89 heads S512 1.05 of the time,
+//   179 heads S199 1.06; in XCD order 102 heads S512 0.94, 160 heads S199 0.91) and, at D = 64, of
+//   rows past 384 or past 7/4 blocks a CU (89 heads S512 1.08, 102 heads 0.93; 253 heads S256 1.07
+//   to 1.29, 179 heads 0.94).
 bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (!eight_wave(a->tile_m, a->tile_n, a->accum, a->D) || a->sched == 3 || ncu <= 0) return false;
   const int64_t S = a->S, n = n_bh * n_qblk;
   if (n <= ncu) return false;
   if (!a->causal) {
+    if (n % 8 != 0 && n <= 2 * (int64_t)ncu && use_rows256(a, n_bh, ncu) && S > 192 * ((S + 255) / 256) &&
+        (a->D == 128 || S > 384 || 4 * n > 7 * (int64_t)ncu))
+      return false;
     if (a->D == 64) return S <= 512 || (S <= 1024 && n >= 4 * (int64_t)ncu);
     return S <= (a->D == 96 ? 1024 : a->D == 128 ? 512 : 768);
   }
@@ -724,12 +737,18 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
     if (S <= 1280) return S <= 768 || (S <= 1024 && n >= 2 * cu) || n225;
     return (n_qblk % 2 == 0 || n > 4 * cu || !pairs_fill(n_bh, n_qblk, ncu)) && ((S <= 1536 && n225) || (S <= 3072 && n375));
   }
-  if (a->D == 160) return S <= 640;
+  const int64_t cu = ncu;
+  if (a->D == 160) return S <= 512 || (S <= 640 && 8 * n >= 9 * cu);
   const bool paired = n >= 2 * (int64_t)ncu;
   const bool full = pairs_fill(n_bh, n_qblk, ncu);
   if (paired && full && n_bh * ((n_qblk + 1) / 2) <= ncu) return false;
-  if (a->D == 128) return S <= 512 || (S <= 640 && paired) || (S <= 768 && paired && !full);
-  return S <= 768 || (S <= 1024 && n > 4 * (int64_t)ncu) || (S <= 1536 && paired && !full);
+  if (a->D == 128) {
+    const bool short_last = paired && 128 * n_qblk - S >= 32;
+    return S <= 512 || (S <= 640 && (short_last || 2 * n >= 5 * cu)) || (S <= 768 && short_last && !full);
+  }
+  if (S <= 768 || (S <= 1024 && n > 4 * cu)) return true;
+  if (S > 1536 || !paired || full) return false;
+  return S <= 1024 || (4 * n >= 9 * cu && (a->D == 64 || n <= 3 * cu));
 }
 
 // Whether input-dtype accumulation on a 128-row tile runs the small-workgroup kernel
