@@ -239,6 +239,12 @@ ta_status ta_describe_launch(const ta_fwd_args* args, int32_t chunk_steps, ta_la
 ta_status ta_describe_launch_model(const ta_fwd_args* args, int32_t chunk_steps,
                                    int32_t compute_units, ta_launch_desc* out);
 
+/* Heads an XCD takes at a time in the whole-row launch of `args` on a device of
+ * `compute_units` CUs (every head's heaviest causal query block before any head's second), 0
+ * where it takes them one after the other.  Reads the same fields as ta_describe_launch; no
+ * counterpart in the reference. */
+ta_status ta_describe_head_group(const ta_fwd_args* args, int32_t compute_units, int32_t* heads);
+
 /* Chunk length meaning "the library's dispatch model decides" (TILEDATTN_SPLIT=auto). */
 #define TA_SPLIT_AUTO (-2)
 

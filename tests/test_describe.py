@@ -351,7 +351,7 @@ def test_policy_defaults_run_the_described_kernels(lib):
     (128, True, 10, 388, True), (128, True, 12, 512, False), (128, True, 16, 512, False),
     (128, True, 14, 640, True), (128, True, 9, 1024, True), (128, True, 9, 1025, False),
     (160, True, 9, 512, True), (160, True, 8, 640, False), (160, True, 10, 640, True),
-    (160, True, 8, 1024, False), (160, True, 9, 1024, True), (160, True, 8, 1536, True),
+    (160, True, 8, 1024, False), (160, True, 9, 1024, True), (160, True, 10, 896, True), (160, True, 8, 1536, True),
     (160, True, 8, 1537, False),
 ])
 def test_small_workgroup_rule(lib, objects, d, causal, b, s, rows):
@@ -439,3 +439,37 @@ def test_small_workgroup_rule_input_dtype_near_one_block_a_cu(lib, d, tn, h, s, 
 def test_small_workgroup_rule_without_xcd_order(lib, d, causal, h, s, rows):
     desc = _d(lib, B=1, H=h, S=s, D=d, causal=causal, tile_m=128, sched=1)
     assert desc.kernel.decode().startswith("ta_fwd_rows_") is rows, desc.kernel
+
+
+@pytest.mark.parametrize("accum", [_lib.TA_ACC_FP32, _lib.TA_ACC_INPUT])
+@pytest.mark.parametrize("d", [64, 96, 128, 160, 256])
+def test_head_groups_are_even_and_bounded(lib, d, accum):
+    """Groups of the causal head order: none below two heads, at most twice plus one the heads (two to
+    eight) whose K and V fit 4 MiB, and no last group of half the others' heads or fewer."""
+    if accum == _lib.TA_ACC_INPUT and d in (96, 160, 256):
+        pytest.skip("no grouped kernel")
+    grouped = 0
+    for heads in range(2, 41):  # a group per XCD
+        for s in (256, 384, 512, 640, 896, 1024, 1152, 1280, 1408, 2048, 2500, 4096):
+            args = _lib.shape_args(B=heads, H=8, S=s, D=d, causal=True, sched=1, accum=accum)
+            g = _lib.head_group(lib, args, CU)
+            if not g:
+                continue
+            grouped += 1
+            fit = min(8, max(2, (4 << 20) // (s * d * 4)))
+            last = heads % g or g
+            assert 2 <= g <= heads and g <= 2 * fit + 1, (heads, s, g, fit)
+            assert 2 * last > g, (heads, s, g)
+    assert grouped > 100
+    for kw in (dict(causal=False), dict(sched=0), dict(H=7)):
+        args = dict(B=20, H=8, S=1024, D=d, causal=True, sched=1, accum=accum)
+        args.update(kw)
+        assert _lib.head_group(lib, _lib.shape_args(**args), CU) == 0
+
+
+@pytest.mark.parametrize("d,heads,s,group", [
+    (256, 56, 1408, 4), (256, 104, 1408, 5), (256, 80, 1152, 5), (256, 40, 2048, 3), (256, 64, 2048, 2),
+    (128, 40, 1000, 5), (160, 48, 1024, 6), (64, 88, 640, 0),
+])
+def test_head_group_sizes(lib, d, heads, s, group):
+    assert _lib.head_group(lib, _lib.shape_args(B=1, H=heads, S=s, D=d, causal=True, sched=1), CU) == group

@@ -58,6 +58,7 @@ EXPORTED_SYMBOLS = (
     "ta_sdpa_fwd_split_static",
     "ta_describe_launch",
     "ta_describe_launch_model",
+    "ta_describe_head_group",
     "ta_plan_call",
     "ta_cache_reset",
     "ta_cache_size",
@@ -170,6 +171,16 @@ def describe(lib: ctypes.CDLL, args: "FwdArgs", chunk_steps: int = 0,
     return out
 
 
+def head_group(lib: ctypes.CDLL, args: "FwdArgs", compute_units: int) -> int:
+    """Heads an XCD takes at a time in the whole-row launch of ``args``
+    (``ta_describe_head_group``); 0: one after the other."""
+    out = ctypes.c_int32(0)
+    st = lib.ta_describe_head_group(ctypes.byref(args), int(compute_units), ctypes.byref(out))
+    if st != TA_OK:
+        raise ValueError(last_error(lib))
+    return int(out.value)
+
+
 _lock = Lock()
 _lib: ctypes.CDLL | None = None
 _call = None
@@ -231,6 +242,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.ta_describe_launch.restype = i32
     lib.ta_describe_launch_model.argtypes = [ctypes.POINTER(FwdArgs), i32, i32, ctypes.POINTER(LaunchDesc)]
     lib.ta_describe_launch_model.restype = i32
+    lib.ta_describe_head_group.argtypes = [ctypes.POINTER(FwdArgs), i32, ctypes.POINTER(i32)]
+    lib.ta_describe_head_group.restype = i32
     lib.ta_plan_call.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, i32, i32, i32,
                                  i32, ctypes.POINTER(CallKnobs), ctypes.POINTER(CallPlan)]
     lib.ta_plan_call.restype = i32

@@ -699,7 +699,7 @@ KernelId pp_d256_kernel_id(int dtype, int causal, int tail) {
 //   D = 128 up to 384, 448 below 1.5 blocks a CU (80 heads S388 15.6 -> 13.0) and 1024 past two
 //   (112 heads S540 27.1 -> 20.6, 96 heads S640 19.2 -> 20.9, 48 heads S1536 37.3 -> 38.6);
 //   D = 160, which has no pairs, up to 512, 768 from 1.5 blocks a CU (96 heads 34.6 -> 30.7,
-//   64 heads S640 20.6 -> 22.6), 1024 from 2.25 (96 heads 46.3 -> 41.2, 48 heads 26.0 -> 28.3)
+//   64 heads S640 20.6 -> 22.6), 1024 past two (80 heads S896 39.3 -> 31.8, 48 heads 26.0 -> 28.3)
 //   and 1536 from three (64 heads 58.1 -> 55.2; 80 heads S1792 1.08 of the time);
 // * causal otherwise: where the pairs of a grid of two blocks a CU or more fill one round of
 //   the CUs only up to S = 384 (D = 64 S512 128 heads 12.8 -> 13.2); else
@@ -731,7 +731,7 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (n_bh % 8 == 0 && a->sched == 1) {
     const int64_t cu = ncu;
     const bool n225 = 4 * n >= 9 * cu, n375 = 4 * n >= 15 * cu;
-    if (a->D == 160) return S <= 512 || (S <= 768 && 2 * n >= 3 * cu) || (S <= 1024 && n225) || (S <= 1536 && n >= 3 * cu);
+    if (a->D == 160) return S <= 512 || (S <= 768 && 2 * n >= 3 * cu) || (S <= 1024 && n > 2 * cu) || (S <= 1536 && n >= 3 * cu);
     if (a->D == 128) return (S <= 448 && 2 * n <= 3 * cu) || (S <= 1024 && n > 2 * cu);
     if (a->D == 96) return S <= 768 || (S <= 960 && n >= 2 * cu) || (S <= 1536 && n225) || (S <= 1920 && n375);
     if (S <= 1280) return S <= 768 || (S <= 1024 && n >= 2 * cu) || n225;
@@ -825,10 +825,12 @@ struct LaunchPlan {
 // CU, which mixes heavy and light by itself: small workgroups, D = 64 96 heads S640 13.4 -> 14.1;
 // with an even number like meets like: 64 heads S1536 31.5 -> 29.6), nor small workgroups of
 // heads of two or three blocks (D = 64 192 heads S200 9.1 -> 9.7).  The heads taken together
-// keep their K and V in the XCD's 4 MiB of L2 (D = 256 64 heads S2048, 2 MiB a head: two at a
-// time 143 us, four 144, eight 150; D = 128 48 heads S1100: two 26.9, six 25.4), two to eight of
-// them, in even groups: a last head by itself starts its heavy block last (D = 256 40 heads
-// S2048 as 2 + 2 + 1 98 -> 111).
+// share the XCD's 4 MiB of L2 for their K and V (D = 256 64 heads S2048, 2 MiB a head: two at a
+// time 143 us, four 144, eight 150; D = 128 48 heads S1100: two 26.9, six 25.4): a group is at
+// most twice, and one more than, the two to eight heads that fit.  Groups are even: a last one of
+// half the others' heads or fewer starts its heavy blocks last (D = 256 56 heads S1408 as 3 + 3 + 1
+// 88.5 us, one by one 76.4, as 4 + 3 68.6; 104 heads S1408 as 4 + 4 + 4 + 1 147, 134, as 5 + 5 + 3
+// 125), so one group fewer is made then.
 int32_t head_group(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int resident, int ncu) {
   if (!a->causal || a->sched != 1 || n_bh % 8 != 0 || n_bh < 16 || ncu < 8) return 0;
   const int64_t heads = n_bh / 8, blocks = heads * n_qblk, cus = ncu / 8;
@@ -837,7 +839,9 @@ int32_t head_group(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int resid
   const int64_t fit = std::min<int64_t>(8, std::max<int64_t>(2, (int64_t{4} << 20) / (a->S * a->D * 4)));
   int64_t groups = std::max<int64_t>(1, heads / fit);
   if (2 * ((heads + groups - 1) / groups) >= 3 * fit && heads % (groups + 1) == 0) ++groups;
-  return static_cast<int32_t>((heads + groups - 1) / groups);
+  auto size = [&] { return (heads + groups - 1) / groups; };
+  while (groups > 1 && 2 * (heads - size() * (groups - 1)) <= size()) --groups;
+  return static_cast<int32_t>(size());
 }
 
 // The plan for shape-validated arguments with n_bh * n_qblk > 0, on a device of `ncu`
@@ -1340,6 +1344,19 @@ ta_status ta_plan_call(int64_t B, int64_t H, int64_t S, int64_t D, int32_t dtype
 ta_status ta_describe_launch_model(const ta_fwd_args* args, int32_t chunk_steps,
                                    int32_t compute_units, ta_launch_desc* out) {
   return describe_model(args, chunk_steps, compute_units, out);
+}
+
+ta_status ta_describe_head_group(const ta_fwd_args* args, int32_t compute_units, int32_t* heads) {
+  if (heads == nullptr) return fail(TA_EINVAL, "heads is NULL");
+  *heads = 0;
+  if (compute_units <= 0) return fail(TA_EINVAL, "compute_units %d", compute_units);
+  int64_t n_bh = 0, n_qblk = 0;
+  ta_status st = validate_args(args, &n_bh, &n_qblk, false);
+  if (st != TA_OK || n_qblk == 0) return st;
+  LaunchPlan pl;
+  st = plan_launch(args, n_bh, n_qblk, 0, compute_units, &pl);
+  if (st == TA_OK) *heads = pl.head_group;
+  return st;
 }
 
 ta_status ta_describe_launch(const ta_fwd_args* args, int32_t chunk_steps, ta_launch_desc* out) {
