@@ -448,7 +448,7 @@ def test_head_groups_are_even_and_bounded(lib, d, accum):
     eight) whose K and V fit 4 MiB, and no last group of half the others' heads or fewer."""
     if accum == _lib.TA_ACC_INPUT and d in (96, 160, 256):
         pytest.skip("no grouped kernel")
-    grouped = 0
+    grouped = few = 0
     for heads in range(2, 41):  # a group per XCD
         for s in (256, 384, 512, 640, 896, 1024, 1152, 1280, 1408, 2048, 2500, 4096):
             args = _lib.shape_args(B=heads, H=8, S=s, D=d, causal=True, sched=1, accum=accum)
@@ -459,8 +459,10 @@ def test_head_groups_are_even_and_bounded(lib, d, accum):
             fit = min(8, max(2, (4 << 20) // (s * d * 4)))
             last = heads % g or g
             assert 2 <= g <= heads and g <= 2 * fit + 1, (heads, s, g, fit)
-            assert 2 * last > g, (heads, s, g)
-    assert grouped > 100
+            # (37 heads: 37 = 4 * 8 + 5 is the first size that leaves more than half)
+            assert 2 * last > g or not any(heads % n == 0 or 2 * (heads % n) > n for n in range(g, 2 * fit + 2)), (heads, s, g)
+            few += heads <= 20 and 2 * last <= g
+    assert grouped > 100 and few == 0
     for kw in (dict(causal=False), dict(sched=0), dict(H=7)):
         args = dict(B=20, H=8, S=1024, D=d, causal=True, sched=1, accum=accum)
         args.update(kw)

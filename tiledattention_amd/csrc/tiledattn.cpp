@@ -830,7 +830,7 @@ struct LaunchPlan {
 // most twice, and one more than, the two to eight heads that fit.  Groups are even: a last one of
 // half the others' heads or fewer starts its heavy blocks last (D = 256 56 heads S1408 as 3 + 3 + 1
 // 88.5 us, one by one 76.4, as 4 + 3 68.6; 104 heads S1408 as 4 + 4 + 4 + 1 147, 134, as 5 + 5 + 3
-// 125), so one group fewer is made then.
+// 125), so larger groups are taken then where the bound has such a size.
 int32_t head_group(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int resident, int ncu) {
   if (!a->causal || a->sched != 1 || n_bh % 8 != 0 || n_bh < 16 || ncu < 8) return 0;
   const int64_t heads = n_bh / 8, blocks = heads * n_qblk, cus = ncu / 8;
@@ -839,9 +839,10 @@ int32_t head_group(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int resid
   const int64_t fit = std::min<int64_t>(8, std::max<int64_t>(2, (int64_t{4} << 20) / (a->S * a->D * 4)));
   int64_t groups = std::max<int64_t>(1, heads / fit);
   if (2 * ((heads + groups - 1) / groups) >= 3 * fit && heads % (groups + 1) == 0) ++groups;
-  auto size = [&] { return (heads + groups - 1) / groups; };
-  while (groups > 1 && 2 * (heads - size() * (groups - 1)) <= size()) --groups;
-  return static_cast<int32_t>(size());
+  const int64_t size = (heads + groups - 1) / groups;
+  for (int64_t g = size; g <= 2 * fit + 1; ++g)
+    if (heads % g == 0 || 2 * (heads % g) > g) return static_cast<int32_t>(g);
+  return static_cast<int32_t>(size);
 }
 
 // The plan for shape-validated arguments with n_bh * n_qblk > 0, on a device of `ncu`
