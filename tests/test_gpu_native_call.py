@@ -104,3 +104,49 @@ def test_library_status_is_raised(gpu):
     finally:
         plan.args.dtype = 0
     sdpa(q, k, v)
+
+
+_WAITER = r"""
+#include <unistd.h>
+extern "C" int flag = 0;
+extern "C" int wait_for_flag(const void*, void*) {  // a ta_sdpa_fwd that blocks, 3 s at most
+  for (int i = 0; i < 3000; ++i) {
+    if (__atomic_load_n(&flag, __ATOMIC_ACQUIRE)) return 0;
+    usleep(1000);
+  }
+  return 4;
+}
+"""
+
+
+def test_other_threads_run_while_the_library_call_blocks(gpu, tmp_path):
+    """The interpreter lock is free during the allocation and the library call, as in the ctypes
+    path: here the call returns only once another Python thread has set its flag."""
+    import ctypes
+    import shutil
+    import subprocess
+    import time
+
+    import torch
+
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not available")
+    (tmp_path / "waiter.cpp").write_text(_WAITER)
+    so = tmp_path / "waiter.so"
+    subprocess.run([gxx, "-O1", "-shared", "-fPIC", "-o", str(so), str(tmp_path / "waiter.cpp")], check=True)
+    waiter = ctypes.CDLL(str(so))
+    flag = ctypes.c_int.in_dll(waiter, "flag")
+    q, k, v = _qkv()
+    plan = _plan(q, k, v, False)
+    say("native call of a library function that waits for another thread")
+
+    def release():
+        time.sleep(0.05)
+        flag.value = 1
+
+    t = threading.Thread(target=release)
+    t.start()
+    out = plan.launch(ctypes.cast(waiter.wait_for_flag, ctypes.c_void_p).value, plan.args_addr, q, k, v, 1.0)
+    t.join()
+    assert isinstance(out, torch.Tensor), f"status {out}: no other thread ran"

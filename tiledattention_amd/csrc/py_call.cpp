@@ -20,6 +20,12 @@ namespace {
 
 using FwdFn = ta_status (*)(const ta_fwd_args*, void*);
 
+// Releases the interpreter lock for a scope (an exception takes it back on its way out).
+struct NoGil {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // launch(function address, ta_fwd_args address, q, k, v, scale) -> the output; None where the
 // arguments are not plain tensors with 16-byte aligned data (the caller copies them then); or
 // the library's status, an int, when it is not TA_OK.
@@ -45,10 +51,17 @@ PyObject* launch(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if ((reinterpret_cast<uintptr_t>(args.q) | reinterpret_cast<uintptr_t>(args.k) |
        reinterpret_cast<uintptr_t>(args.v)) & 15)
     Py_RETURN_NONE;
-  at::Tensor out = at::empty(q.sizes(), q.options());
-  args.o = out.data_ptr();
   args.scale = static_cast<float>(scale);
-  const ta_status st = fn(&args, c10::hip::getCurrentHIPStream(q.device().index()).stream());
+  at::Tensor out;
+  ta_status st;
+  {
+    // Other threads run meanwhile, as during torch's own calls and a ctypes one: the allocation
+    // may wait for the device, the first launch loads a module, and a full queue blocks.
+    const NoGil no_gil;
+    out = at::empty(q.sizes(), q.options());
+    args.o = out.data_ptr();
+    st = fn(&args, c10::hip::getCurrentHIPStream(q.device().index()).stream());
+  }
   if (st != TA_OK) return PyLong_FromLong(st);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
