@@ -81,6 +81,23 @@ def test_missing_code_object_is_a_dependency_error(monkeypatch: pytest.MonkeyPat
         _lib.load()
 
 
+@pytest.mark.parametrize("content", [None, b"", b"not an extension module"])
+def test_call_module_is_optional(monkeypatch: pytest.MonkeyPatch, tmp_path, content) -> None:
+    # Absent, empty or built for something else: no module, and no error.
+    import sysconfig
+
+    from tiledattention import _lib
+
+    monkeypatch.setenv("TILEDATTN_LIB_DIR", str(tmp_path))
+    monkeypatch.setattr(_lib, "_call", None)
+    path = _lib.call_module_path()
+    assert path.parent == tmp_path and path.name == "_tiledattn_call" + sysconfig.get_config_var("EXT_SUFFIX")
+    (tmp_path / "_tiledattn_call.cpython-00-other.so").write_bytes(b"")  # another Python's: never looked at
+    if content is not None:
+        path.write_bytes(content)
+    assert _lib.load_call() is None and _lib.loaded_call() is None
+
+
 def test_gate_passes_with_fakes_and_is_cached(monkeypatch: pytest.MonkeyPatch) -> None:
     import tiledattention._runtime as runtime
 

@@ -106,6 +106,25 @@ def test_library_status_is_raised(gpu):
     sdpa(q, k, v)
 
 
+def test_calls_work_without_the_module(gpu, monkeypatch, tmp_path):
+    """A library directory without the module: the ctypes path launches the same kernel."""
+    import torch
+
+    from tiledattention import _lib, sdpa
+    from tiledattention.kernels import flash_fwd
+
+    q, k, v = _qkv((1, 3, 130, 64))
+    want = sdpa(q, k, v, causal=True)
+    monkeypatch.setattr(_lib, "call_module_path", lambda: tmp_path / "absent.so")
+    monkeypatch.setattr(_lib, "_call", None)
+    monkeypatch.setattr(flash_fwd, "_PLANS", {})
+    monkeypatch.setattr(flash_fwd, "_PLANS_BY_LAYOUT", {})
+    say("ctypes call without the native module")
+    for _ in range(2):
+        assert torch.equal(sdpa(q, k, v, causal=True), want)
+    assert _plan(q, k, v, True).launch is None and _lib.loaded_call() is None
+
+
 _WAITER = r"""
 #include <unistd.h>
 extern "C" int flag = 0;

@@ -38,6 +38,9 @@ def test_layout_mirrors_the_package(package):
     assert got == src | {kb.Path("_ops.py")}
     assert (pkg / "lib" / "libtiledattn.so").exists()
     assert {p.name for p in (pkg / "lib").glob("*.hsaco")} == {p.name for p in kb.LIB_SRC.glob("*.hsaco")}
+    # the call module under the name of the Python it was built for only
+    names = {p.name for p in (pkg / "lib").glob("_tiledattn_call*")}
+    assert names == {p.name for p in kb.LIB_SRC.glob("_tiledattn_call.*.so")} and _lib.call_module_path().name in names
     # rewriting replaces the tree
     again = kb.write_kernel_package(root / "build")
     assert again == pkg and (pkg / "_ops.py").exists()

@@ -4,7 +4,8 @@ The library and the gfx950 code objects it loads are built in-tree by
 ``tiledattention_amd/csrc/build.py`` into ``tiledattention_amd/lib/`` (the native package
 beside this one; located without importing it).  ``TILEDATTN_LIB_DIR`` overrides where both
 are looked up.  Nothing here falls back to another implementation: if the library is
-missing, ``load()`` raises ``DependencyError``.
+missing, ``load()`` raises ``DependencyError``.  (``load_call()``'s module only shortens the
+way from a Python call to the same library call.)
 """
 
 from __future__ import annotations
@@ -12,6 +13,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import sysconfig
 from pathlib import Path
 from threading import Lock
 
@@ -290,31 +292,33 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+def call_module_path() -> Path:
+    """The module's file: its name carries the CPython ABI, so another Python never loads it."""
+    return lib_dir() / f"_tiledattn_call{sysconfig.get_config_var('EXT_SUFFIX')}"
+
+
 def load_call():
     """The CPython module ``_tiledattn_call`` beside the library (``launch``: a planned call's
-    allocation and launch), loaded once per process; ``DependencyError`` if absent."""
+    allocation and launch), loaded once per process.  None where it is absent, built for another
+    Python or not importable beside this torch: calls then take the ctypes path, which launches
+    the same kernels."""
     global _call
     with _lock:
         if _call is None:
-            path = lib_dir() / "_tiledattn_call.so"
-            if not path.exists():
-                raise DependencyError(
-                    f"Native call module {path} is missing. Build it with "
-                    "`python -m tiledattention_amd.csrc.build`."
-                )
+            path = call_module_path()
             try:
                 spec = importlib.util.spec_from_file_location("_tiledattn_call", path)
                 mod = importlib.util.module_from_spec(spec)
                 spec.loader.exec_module(mod)
-            except ImportError as exc:
-                raise DependencyError(f"Native call module {path} could not be loaded: {exc}") from exc
+            except (ImportError, OSError):
+                mod = False
             _call = mod
-        return _call
+        return _call or None
 
 
 def loaded_call():
     """``_tiledattn_call`` if ``load_call()`` already succeeded in this process, else None."""
-    return _call
+    return _call or None
 
 
 def loaded() -> ctypes.CDLL | None:

@@ -724,10 +724,11 @@ def _build_plan(torch_mod, lib, q, k, v, causal: bool, tile: tuple[int, int] | N
     plan.ws_bytes = pol.ws_bytes
     plan.args = args
     # A call of plain tensors that launches one kernel over inputs read in place, without a
-    # sync mode, goes from its plan to the launch natively (_tiledattn_call).
-    if (type(q) is torch_mod.Tensor and plan.out_like_q and sync_mode == "async" and not plan.ws_bytes
-            and not any(plan.copy)):
-        plan.launch = _lib.load_call().launch
+    # sync mode, goes from its plan to the launch natively (_tiledattn_call, where it is there).
+    call = _lib.load_call()
+    if (call is not None and type(q) is torch_mod.Tensor and plan.out_like_q and sync_mode == "async"
+            and not plan.ws_bytes and not any(plan.copy)):
+        plan.launch = call.launch
         plan.fn_addr = ctypes.cast(lib.ta_sdpa_fwd, ctypes.c_void_p).value
         plan.args_addr = ctypes.addressof(args)
     return plan

@@ -14,8 +14,8 @@ Outputs (into ``tiledattention_amd/lib/`` unless told otherwise):
   ``ta_sdpa_fwd_split_static``);
 * ``libtiledattn_torch.so``: the C++ torch operator ``tiledattention::sdpa_fwd``
   (``torch_ext.cpp``, g++ against the installed torch), linked to ``libtiledattn.so``;
-* ``_tiledattn_call.so``: the native tail of a Python call (``py_call.cpp``, a CPython
-  extension module over the installed torch).
+* ``_tiledattn_call.<CPython ABI>.so``: the native tail of a Python call (``py_call.cpp``, a
+  CPython extension module over the installed torch; calls work without it).
 
 Run as ``python -m tiledattention_amd.csrc.build``.
 """
@@ -191,7 +191,7 @@ def py_call_cmd(out_dir: Path) -> list[str]:
         f"-I{ROCM / 'include'}",
         f"-I{REPO / 'include'}",
         "-o",
-        str(out_dir / "_tiledattn_call.so"),
+        str(out_dir / f"_tiledattn_call{sysconfig.get_config_var('EXT_SUFFIX')}"),
         str(HERE / "py_call.cpp"),
         f"-L{tlib}",
         f"-Wl,-rpath,{tlib}",

@@ -77,7 +77,7 @@ def write_kernel_package(out: Path, variant: str | None = None) -> Path:
     """Lay the kernel package out under ``out/<variant>/tiledattention`` (replacing a previous
     one) and return that directory."""
     lib_files = (sorted(LIB_SRC.glob("libtiledattn.so")) + sorted(LIB_SRC.glob("libtiledattn_torch.so"))
-                 + sorted(LIB_SRC.glob("_tiledattn_call.so")) + sorted(LIB_SRC.glob("*.hsaco")))
+                 + sorted(LIB_SRC.glob("_tiledattn_call.*.so")) + sorted(LIB_SRC.glob("*.hsaco")))
     if not any(f.name == "libtiledattn.so" for f in lib_files):
         raise FileNotFoundError(
             f"{LIB_SRC}/libtiledattn.so is missing: build it first (python -m tiledattention_amd.csrc.build)"
