@@ -106,6 +106,28 @@ def test_library_status_is_raised(gpu):
     sdpa(q, k, v)
 
 
+def test_plan_made_by_another_tensor_type(gpu, monkeypatch):
+    """The first call of a layout with a Parameter, or a subclass, as q: later plain calls are
+    native all the same."""
+    import torch
+
+    from tiledattention import sdpa
+    from tiledattention.kernels import flash_fwd
+
+    class Sub(torch.Tensor):
+        pass
+
+    q, k, v = _qkv((1, 3, 140, 64))
+    want = sdpa(q, k, v, causal=True)
+    for first in (torch.nn.Parameter(q, requires_grad=False), torch.nn.Parameter(q), q.as_subclass(Sub)):
+        monkeypatch.setattr(flash_fwd, "_PLANS", {})
+        monkeypatch.setattr(flash_fwd, "_PLANS_BY_LAYOUT", {})
+        say(f"plan made by {type(first).__name__}")
+        out = sdpa(first, k, v, causal=True)
+        assert torch.equal(out.as_subclass(torch.Tensor), want) and not out.requires_grad
+        assert _plan(q, k, v, True).launch is not None and torch.equal(sdpa(q, k, v, causal=True), want)
+
+
 def test_calls_work_without_the_module(gpu, monkeypatch, tmp_path):
     """A library directory without the module: the ctypes path launches the same kernel."""
     import torch

@@ -723,11 +723,12 @@ def _build_plan(torch_mod, lib, q, k, v, causal: bool, tile: tuple[int, int] | N
     plan.chunk = pol.chunk
     plan.ws_bytes = pol.ws_bytes
     plan.args = args
-    # A call of plain tensors that launches one kernel over inputs read in place, without a
-    # sync mode, goes from its plan to the launch natively (_tiledattn_call, where it is there).
+    # A call that launches one kernel over inputs read in place, without a sync mode, goes from
+    # its plan to the launch natively (_tiledattn_call, where it is there).  The plan serves every
+    # tensor of its layout, whatever the type of the first: launch() itself leaves the ones it
+    # does not take (subclasses other than Parameter) to the path below.
     call = _lib.load_call()
-    if (call is not None and type(q) is torch_mod.Tensor and plan.out_like_q and sync_mode == "async"
-            and not plan.ws_bytes and not any(plan.copy)):
+    if call is not None and plan.out_like_q and sync_mode == "async" and not plan.ws_bytes and not any(plan.copy):
         plan.launch = call.launch
         plan.fn_addr = ctypes.cast(lib.ta_sdpa_fwd, ctypes.c_void_p).value
         plan.args_addr = ctypes.addressof(args)

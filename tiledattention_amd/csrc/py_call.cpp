@@ -26,6 +26,8 @@ struct NoGil {
   ~NoGil() { PyEval_RestoreThread(state); }
 };
 
+// (Plain tensors below: torch.Tensor and torch.nn.Parameter, THPVariable_CheckExact.)
+//
 // launch(function address, ta_fwd_args address, q, k, v, scale) -> the output; None where the
 // arguments are not plain tensors with 16-byte aligned data (the caller copies them then); or
 // the library's status, an int, when it is not TA_OK.
@@ -67,7 +69,7 @@ PyObject* launch(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// The three arguments as tensors, when each is a plain torch.Tensor.
+// The three arguments as tensors, when each is a plain tensor.
 bool plain(PyObject* const* a, Py_ssize_t n, const at::Tensor** t) {
   if (n != 3) return false;
   for (int i = 0; i < 3; ++i) {
