@@ -5,7 +5,9 @@ bf16, causal, seed 1234, default knobs.  A "step" is one forward over that batch
 inputs already resident in HBM.  Work per step is 4*B*H*S^2*D FLOPs halved for causal
 (137.4 GFLOP), so ``value`` is TFLOP/s.
 
-The JSON line also carries:
+The JSON line is the headline alone, below ``LINE_MAX`` characters, with ``roofline``,
+``cpu_baseline`` and the TFLOP/s of ``sweep``.  What else is measured goes to stderr as it is
+measured, and with ``--detail-json FILE`` to that file, as one JSON record of the line with:
 
 * ``roofline``: the attention kernel's achieved TFLOP/s (algorithmic FLOPs per launch /
   mean launch duration: two HIP events on the launch stream around the timed region's K
@@ -14,7 +16,7 @@ The JSON line also carries:
   rocprofv3 counters (profiles/), or null when not measured in this run;
 * ``cpu_baseline``: the reference's eager attention restated on the host CPU
   (oracle/eager.py, run_study.py:304-335) on a bounded sample of the same workload;
-* ``sweep``: the C3 sequence sweep S in {512..8192} (bf16), as before;
+* ``sweep``: the C3 sequence sweep S in {512..8192} (bf16);
 * ``blocks``: every other BASELINE.json configuration, each timed the same way (TFLOP/s,
   share of peak, algorithmic HBM GB/s, mean and p95 per call, the kernel the library
   launches): C2, the C4 tile x accumulation sweep (fp16/bf16, D 64/128), C5 and its outlier
@@ -31,7 +33,7 @@ Inputs are generated on the CPU from a seeded ``torch.Generator`` (q, k, v drawn
 order, as run_study.py:526-529 does) and copied to the GPU before any timing.
 
 Usage: ``python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-cpu-baseline]
-[--no-sweep] [--no-blocks] [--only-block NAME]``.
+[--no-sweep] [--no-blocks] [--only-block NAME] [--detail-json FILE]``.
 """
 
 from __future__ import annotations
@@ -50,6 +52,7 @@ if str(ROOT) not in sys.path:
     sys.path.insert(0, str(ROOT))
 
 PEAK_TFLOPS = 2516.6  # dense fp16/bf16 MFMA, MI355X: 256 CU * 4096 FLOP/clk * 2.4 GHz
+LINE_MAX = 4000  # a reader of the output's last few KB gets the whole line
 REFERENCE_GB10_C3_S8192 = 60.87  # benchmark-gb10/results/benchmark_results.csv:548, TFLOP/s
 C4_TILES = ((64, 64), (64, 128), (128, 64), (128, 128))
 GRID_S = (512, 1024, 2048, 4096, 8192)
@@ -89,6 +92,7 @@ def _args():
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-sweep", action="store_true")
     ap.add_argument("--no-blocks", action="store_true", help="skip the other BASELINE configurations")
+    ap.add_argument("--detail-json", default="", help="write the whole record (sweep, blocks) to this file")
     ap.add_argument("--only-block", default="", help="run only blocks whose name starts with this")
     ap.add_argument("--traffic-json", default=str(ROOT / "profiles" / "traffic.json"),
                     help="HBM bytes per launch measured by rocprofv3 (optional)")
@@ -491,6 +495,13 @@ def cpu_baseline(shape, dtype: str, seed: int, causal: bool, budget_s: float):
     }
 
 
+def headline(record: dict) -> dict:
+    """The record as the printed line has it: no blocks, of the sweep the TFLOP/s only."""
+    line = {k: v for k, v in record.items() if k != "blocks"}
+    line["sweep"] = {s: rec["tflops"] for s, rec in record["sweep"].items()}
+    return line
+
+
 def main() -> int:
     args = _args()
     if args.gpus != 1:
@@ -604,7 +615,9 @@ def main() -> int:
     else:
         line["cpu_baseline"] = None
 
-    print(json.dumps(line), flush=True)
+    if args.detail_json:
+        Path(args.detail_json).write_text(json.dumps(line) + "\n")
+    print(json.dumps(headline(line)), flush=True)
     return 0
 
 

@@ -107,3 +107,28 @@ def test_bench_small_block_stays_in_the_planned_range():
         assert 2 * bh * -(-s // 64) <= 256, (bh, s)
     names = {"TILEDATTN_" + k.upper() for _, env in bench.SMALL_ALTERNATIVES for k in env}
     assert names <= set(flash_fwd._KNOBS)
+
+
+def test_bench_line_is_short_and_keeps_the_headline():
+    """The printed line of a full record: every headline key, the sweep's rates, no blocks, and
+    short enough for a reader of the output's tail."""
+    import json
+
+    sys.path.insert(0, str(ROOT))
+    import bench
+
+    point = {"tflops": 1169.893, "frac_peak": 0.4649, "hbm_gbs": 571.0, "mean_ms": 0.11748, "p95_ms": 0.1199,
+             "kernel": "ta_fwd_pp_pair_bf16_d128_c1_t0"}
+    desc = {f"field_{i}": "ta_fwd_pp_pair_bf16_d128_c1_t0" for i in range(18)}
+    keys = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+            "vs_baseline", "dtype", "data")
+    record = {k: "x" * 90 for k in keys}
+    record["config"] = {"launch": desc, "workload": "x" * 90}
+    record["roofline"] = {f"r{i}": 123456.789 for i in range(8)}
+    record["cpu_baseline"] = {f"c{i}": "x" * 30 for i in range(9)}
+    record["sweep"] = {str(s): point for s in bench.GRID_S}
+    record["blocks"] = {f"block{i}": point for i in range(150)}
+    line = bench.headline(record)
+    assert set(line) == set(record) - {"blocks"} and line["sweep"] == {str(s): 1169.893 for s in bench.GRID_S}
+    assert {k: line[k] for k in keys} == {k: record[k] for k in keys}
+    assert len(json.dumps(line)) < bench.LINE_MAX < len(json.dumps(record))
