@@ -363,13 +363,21 @@ def test_small_workgroup_rule(lib, objects, d, causal, b, s, rows):
             assert desc.kernel.decode() == f"ta_fwd_rows_bf16_d{d}_c{int(causal)}_t{int(not (aligned and s % 128 == 0))}"
             assert (desc.grid, desc.block, desc.rows) == (8 * b * -(-s // 128), 256, 128)
             assert desc.layout == _lib.TA_LAYOUT_WHOLE_ROWS
-    # forced pairs, 64-row tiles and input-dtype accumulation keep their kernels
-    for kw in (dict(sched=3), dict(tile_m=64), dict(accum=_lib.TA_ACC_INPUT)):
-        if d == 96 and "accum" in kw or d == 160 and "accum" in kw:
-            continue
+    # Forced pairs and 64-row tiles keep the eight-wave kernels (the wide one on small grids, which
+    # these are not).
+    for kw, prefix in ((dict(sched=3), "ta_fwd_pp"), (dict(tile_m=64), "ta_fwd_pp64_")):
         args = dict(B=b, H=8, S=s, D=d, causal=causal, tile_m=128, sched=1)
         args.update(kw)
-        assert not _d(lib, **args).kernel.decode().startswith("ta_fwd_rows_")
+        assert _d(lib, **args).kernel.decode().startswith(prefix)
+    # Input-dtype accumulation has its own small workgroups, by a rule of its own.
+    if d in (64, 128):
+        desc = _d(lib, B=b, H=8, S=s, D=d, causal=causal, tile_m=128, sched=1, accum=_lib.TA_ACC_INPUT)
+        n = 8 * b * -(-s // 128)
+        line = 512 if not causal else 3072 if d == 64 and n >= 6 * CU else 2048 if n >= 3 * CU else 1024
+        free = not causal and (d == 64 or s <= 4096)
+        near_one = causal and s > 512 and (n * 3 <= 4 * CU if -(-s // 128) == 7 else n * 8 < 9 * CU if d == 64 else n * 4 < 5 * CU)
+        fam = "rowsl" if n > CU and (free or (causal and s <= line and not (s <= 1024 and near_one))) else "ppl"
+        assert desc.kernel.decode() == f"ta_fwd_{fam}_n64_bf16_d{d}_c{int(causal)}_t{int(s % 128 != 0)}"
 
 
 # Heads that the XCDs cannot take whole: small workgroups and pairs by the grid's size alone.
@@ -441,13 +449,11 @@ def test_small_workgroup_rule_without_xcd_order(lib, d, causal, h, s, rows):
     assert desc.kernel.decode().startswith("ta_fwd_rows_") is rows, desc.kernel
 
 
-@pytest.mark.parametrize("accum", [_lib.TA_ACC_FP32, _lib.TA_ACC_INPUT])
-@pytest.mark.parametrize("d", [64, 96, 128, 160, 256])
+@pytest.mark.parametrize("d,accum", [(d, _lib.TA_ACC_FP32) for d in (64, 96, 128, 160, 256)]
+                         + [(d, _lib.TA_ACC_INPUT) for d in (64, 128)])
 def test_head_groups_are_even_and_bounded(lib, d, accum):
     """Groups of the causal head order: none below two heads, at most twice plus one the heads (two to
     eight) whose K and V fit 4 MiB, and no last group of half the others' heads or fewer."""
-    if accum == _lib.TA_ACC_INPUT and d in (96, 160, 256):
-        pytest.skip("no grouped kernel")
     grouped = few = 0
     for heads in range(2, 41):  # a group per XCD
         for s in (256, 384, 512, 640, 896, 1024, 1152, 1280, 1408, 2048, 2500, 4096):

@@ -8,8 +8,10 @@ finite.  One case is implementation-defined: a NaN in a value row j under the ca
 The oracle computes row i over its visible keys only (rows i >= j are NaN); a tiled kernel
 multiplies the masked keys' P = 0 by V inside the diagonal tile, and 0 x NaN = NaN, so here
 every row of the query block holding j is NaN as well, from the block's first row on (128
-rows for the 128-row and 64-row kernels, whose diagonal key step is 128 keys; 32 for the
-wide kernel's blocks; the reference's tiled kernel does the same at its own tile size; its
+rows for the 128-row and 64-row kernels, whose diagonal key step is 128 keys, and for the
+eight-wave kernel at D = 256; 32 for the wide kernel's blocks; in the small workgroups, whose
+waves of 32 rows walk key tiles of 64 by themselves, every row from j's tile on; the reference's
+tiled kernel does the same at its own tile size; its
 eager baseline, which multiplies the full masked P, makes every row NaN).  That case is
 checked against exactly that rule, with the block size of the kernel that ran."""
 
@@ -73,3 +75,33 @@ def test_nonfinite_propagation(gpu, tensor, row, value, causal):
         out = run_gpu(q, k, v, causal=causal, split=split, accum_mode="fp32")
         _compare(as_f32(out), ref, "bfloat16", f"{tensor} row {row} = {value} causal={causal} split={split}",
                  nan_from_row=nan_from)
+
+
+@pytest.mark.parametrize("tensor,row,value", [
+    ("q", 37, float("nan")), ("k", 200, float("nan")), ("v", 200, float("nan")), ("k", 5, float("inf")),
+    ("v", 299, float("inf")),
+])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("shape,kernel,block", [
+    ((1, 2, 300, 256), "ta_fwd_pp_bf16_d256", 128),
+    ((12, 8, 300, 64), "ta_fwd_rows_bf16_d64", 64),
+    ((12, 8, 300, 96), "ta_fwd_rows_bf16_d96", 64),
+])
+def test_nonfinite_propagation_d256_and_small_workgroups(gpu, shape, kernel, block, tensor, row, value, causal):
+    t3 = dict(zip("qkv", inputs(shape, "bfloat16", 98)))
+    t3[tensor] = _poison(t3[tensor], row, value)
+    q, k, v = t3.values()
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = oracle_f32(q, k, v, causal=causal)
+    assert not np.isfinite(ref).all()
+    name = kernel_for(q, k, v, causal=causal)
+    assert name.startswith(kernel), name
+    say(f"non-finite {tensor}[0,1,{row},:]={value} causal={causal} kernel={name}")
+    got = as_f32(run_gpu(q, k, v, causal=causal))
+    masked = causal and tensor == "v"  # 0 x NaN and 0 x inf: NaN from the key's block or tile on
+    if masked and value == float("inf"):
+        first = row // block * block
+        assert np.isnan(got[0, 1, first:row]).all() and not np.isfinite(got[0, 1, row:]).any()
+        ref[0, 1, first:], got[0, 1, first:] = 0.0, 0.0
+    _compare(got, ref, "bfloat16", f"{kernel} {tensor} row {row} = {value} causal={causal}",
+             nan_from_row=row // block * block if masked and value != float("inf") else None)
