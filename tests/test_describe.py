@@ -375,7 +375,7 @@ def test_small_workgroup_rule(lib, objects, d, causal, b, s, rows):
         n = 8 * b * -(-s // 128)
         line = 512 if not causal else 3072 if d == 64 and n >= 6 * CU else 2048 if n >= 3 * CU else 1024
         free = not causal and (d == 64 or s <= 4096)
-        near_one = causal and s > 512 and (n * 3 <= 4 * CU if -(-s // 128) == 7 else n * 8 < 9 * CU if d == 64 else n * 4 < 5 * CU)
+        near_one = causal and s > 512 and (n * 3 <= 4 * CU if -(-s // 128) == 7 else n * 8 < 9 * CU and -s % 128 < 64)
         fam = "rowsl" if n > CU and (free or (causal and s <= line and not (s <= 1024 and near_one))) else "ppl"
         assert desc.kernel.decode() == f"ta_fwd_{fam}_n64_bf16_d{d}_c{int(causal)}_t{int(s % 128 != 0)}"
 
@@ -416,11 +416,12 @@ def test_small_workgroup_rule_input_dtype(lib, objects, d, tn, causal, b, s, row
 
 # Just above one block per CU a causal grid of longer rows keeps the eight-wave kernel.
 @pytest.mark.parametrize("d,tn,h,s,rows", [
-    (64, 64, 65, 512, True), (64, 64, 52, 640, False), (64, 128, 64, 640, True),
+    (64, 64, 65, 512, True), (64, 64, 56, 533, True), (64, 64, 52, 576, True), (64, 64, 52, 577, False),
+    (64, 64, 52, 640, False), (64, 128, 64, 640, True),
     (64, 64, 47, 768, False), (64, 64, 48, 768, True), (64, 128, 40, 896, False), (64, 64, 48, 896, False),
-    (64, 64, 49, 896, True), (64, 128, 35, 1024, False), (64, 64, 36, 1024, True),
+    (64, 64, 49, 896, True), (64, 128, 39, 1024, False), (64, 64, 40, 1024, True), (128, 64, 48, 768, True),
     (128, 64, 65, 512, True), (128, 64, 56, 640, False), (128, 64, 64, 640, True), (128, 64, 53, 768, False),
-    (128, 64, 40, 834, False), (128, 64, 48, 896, False), (128, 64, 49, 896, True),
+    (128, 64, 40, 776, False), (128, 64, 40, 834, False), (128, 64, 48, 896, False), (128, 64, 49, 896, True),
     (128, 64, 39, 1024, False), (128, 64, 40, 1024, True),
 ])
 def test_small_workgroup_rule_input_dtype_near_one_block_a_cu(lib, d, tn, h, s, rows):
@@ -439,7 +440,8 @@ def test_small_workgroup_rule_input_dtype_near_one_block_a_cu(lib, d, tn, h, s, 
     (128, False, 65, 512, False), (128, False, 102, 512, True), (128, False, 179, 199, False),
     (128, False, 160, 199, True), (128, False, 179, 192, True), (128, False, 100, 330, True), (128, False, 257, 256, True),
     (64, True, 58, 1152, False), (64, True, 71, 1152, True), (64, True, 58, 1024, False), (96, True, 58, 1152, False),
-    (96, True, 71, 1152, True), (96, True, 53, 1536, True), (96, True, 67, 1536, False), (64, True, 67, 1536, True),
+    (96, True, 57, 1088, True), (96, True, 57, 1089, False), (96, True, 71, 1152, True), (96, True, 53, 1536, True),
+    (96, True, 67, 1536, False), (64, True, 67, 1536, True),
     (128, True, 105, 576, True), (128, True, 105, 640, False), (128, True, 105, 609, False), (128, True, 107, 711, True),
     (128, True, 107, 736, True), (128, True, 107, 768, False),
     (160, True, 52, 640, False), (160, True, 58, 640, True), (160, True, 65, 512, True),

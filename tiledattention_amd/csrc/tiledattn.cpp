@@ -748,7 +748,7 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   }
   if (S <= 768 || (S <= 1024 && n > 4 * cu)) return true;
   if (S > 1536 || !paired || full) return false;
-  return S <= 1024 || (4 * n >= 9 * cu && (a->D == 64 || n <= 3 * cu));
+  return S <= 1024 || ((4 * n >= 9 * cu || 128 * n_qblk - S >= 64) && (a->D == 64 || n <= 3 * cu));
 }
 
 // Whether input-dtype accumulation on a 128-row tile runs the small-workgroup kernel
@@ -761,11 +761,13 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
 //   two, TILE_N 128 43.0 -> 42.9) and 3072 from six (64 heads 155 -> 130; S4096 32 heads fp16
 //   127 -> 130);
 // * causal, S = 513 to 1024: not just above one block a CU, where most CUs hold a single small
-//   workgroup, half as fast as an eight-wave one: from 9/8 blocks a CU at D = 64 (TILE_N 128, 35
-//   heads S1024 22.6 -> 23.1; 48 heads S768 0.86 of the time), 5/4 at D = 128 (fp16 56 heads S640
-//   18.9 -> 21.1, 33 heads S1024 34.7 -> 37.5; 64 heads S640 0.98, 40 heads S1024 0.79), and past
-//   4/3 for heads of seven blocks (D = 128 40 heads S834 21.5 -> 25.0, 48 heads S896 27.7 -> 30.8,
-//   D = 64 TILE_N 128 40 heads S896 13.7 -> 15.6; 55 heads 0.92 and 0.86);
+//   workgroup, half as fast as an eight-wave one.  Whole heads on every XCD from 9/8 blocks a CU
+//   (fp16 D = 128 56 heads S640 18.9 -> 21.1; 48 heads S768 0.96 of the time, 40 heads S1024 0.79),
+//   heads of seven blocks, which are not grouped there, past 4/3 (40 heads S834 21.5 -> 25.0, 48
+//   heads S896 27.7 -> 30.8; 56 heads 0.96); others from 5/4 (39 heads S1024 35.9 -> 38.9, D = 64
+//   TILE_N 128 23.3 -> 24.0; 46 heads S896 0.99, 54 heads S768 0.95).  With 64 rows or more missing
+//   from the last block, which they skip, the small workgroups keep all but the heads of seven
+//   blocks (D = 64 56 heads S533 15.5 -> 12.9, D = 128 40 heads S776 20.6 -> 22.6);
 // * D = 128, TILE_N 64: non-causal up to S = 4096 (16 heads 158 -> 149), causal as D = 64 to
 //   2048 (64 heads 119 -> 109, S3072 32 heads 116 -> 124); TILE_N 128, half the rounding:
 //   non-causal up to 768 (128 heads 51.0 -> 49.2, S1024 64 heads 41.4 -> 41.4), causal up to
@@ -778,7 +780,10 @@ bool use_rowsl(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (!a->causal) return a->D == 64 || S <= 4096;
   const int64_t cu = ncu;
   if (S <= 512) return true;
-  if (S <= 1024) return n_qblk == 7 ? 3 * n > 4 * cu : a->D == 64 ? 8 * n >= 9 * cu : 4 * n >= 5 * cu;
+  if (S <= 1024) {
+    if (n_bh % 8 == 0 && n_qblk == 7) return 3 * n > 4 * cu;
+    return 128 * n_qblk - S >= 64 || (n_bh % 8 != 0 ? 4 * n >= 5 * cu : 8 * n >= 9 * cu);
+  }
   return (S <= 2048 && n >= 3 * cu) || (a->D == 64 && S <= 3072 && n >= 6 * cu);
 }
 
