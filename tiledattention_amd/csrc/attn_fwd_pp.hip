@@ -1254,8 +1254,8 @@ __device__ __forceinline__ void attn_fwd_pp_body(const FwdParams& p) {
     constexpr bool GROUPED = CAUSAL && TMR == 128 && LOWP_TN == 0 && !SPLIT;
     // There the addresses and strides are loaded ahead of the numbering's divisions; the compiler
     // would sink these loads into its branches, behind them (B1 H128 S192 D128 causal 8.7 ->
-    // 9.0 us).
-    if constexpr (GROUPED) {
+    // 9.0 us).  Not at D = 64, where it measured slower (fp16 H40 S1005 causal 14.6 -> 15.0).
+    if constexpr (GROUPED && D != 64) {
       asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.o), "s"(p.q_sb), "s"(p.q_sh), "s"(p.q_ss), "s"(p.k_sb),
                    "s"(p.k_sh), "s"(p.k_ss), "s"(p.v_sb), "s"(p.v_sh), "s"(p.v_ss), "s"(p.o_sb), "s"(p.o_sh),
                    "s"(p.o_ss));

@@ -348,6 +348,9 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
     }
     tile(t, k_cur, v_cur, par_tag);
   };
+  // The loop starts at a multiple of 32 bytes, whatever the prologue's length: D = 64 non-causal
+  // B8 H12 S448 11.4 us here, 11.6 twenty bytes further on (S320 1.3 %, S512 1 %).
+  asm volatile(".p2align 5");
   for (int t = 0; t < n_tiles; t += 2) {
     step(t, lds_k0, lds_v0, lds_k1, lds_v1, std::integral_constant<int, 0>{});
     if (t + 1 < n_tiles) step(t + 1, lds_k1, lds_v1, lds_k0, lds_v0, std::integral_constant<int, 1>{});
