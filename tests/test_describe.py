@@ -437,7 +437,7 @@ def test_small_workgroup_rule_input_dtype_near_one_block_a_cu(lib, d, tn, h, s, 
 @pytest.mark.parametrize("d,causal,h,s,rows", [
     (64, False, 65, 512, False), (64, False, 66, 512, True), (64, False, 89, 449, False), (64, False, 102, 512, True),
     (64, False, 129, 512, True), (64, False, 179, 256, True), (64, False, 253, 256, False), (64, False, 89, 384, True),
-    (128, False, 65, 512, False), (128, False, 102, 512, True), (128, False, 179, 199, False),
+    (128, False, 65, 512, False), (128, False, 102, 512, True), (128, False, 179, 199, False), (128, False, 221, 243, True),
     (128, False, 160, 199, True), (128, False, 179, 192, True), (128, False, 100, 330, True), (128, False, 257, 256, True),
     (64, True, 58, 1152, False), (64, True, 71, 1152, True), (64, True, 58, 1024, False), (96, True, 58, 1152, False),
     (96, True, 57, 1088, True), (96, True, 57, 1089, False), (96, True, 71, 1152, True), (96, True, 53, 1536, True),

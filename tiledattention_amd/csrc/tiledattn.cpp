@@ -712,8 +712,9 @@ KernelId pp_d256_kernel_id(int dtype, int causal, int tail) {
 //   D = 160 up to 512, 640 from 9/8 blocks a CU (52 heads 23.3 -> 24.2);
 // * non-causal grids that the XCDs cannot share evenly (n not a multiple of 8: both kernels then
 //   take heads in plain order, which costs the small workgroups more), one round of 256-row blocks
-//   whose rows are more than three quarters real: those at D = 128 (89 heads S512 1.05 of the time,
-//   179 heads S199 1.06; in XCD order 102 heads S512 0.94, 160 heads S199 0.91) and, at D = 64, of
+//   whose rows are more than three quarters real: those at D = 128, but for rows of 225 to 256 (89
+//   heads S512 1.05 of the time, 179 heads S199 1.06, 221 heads S243 0.95; in XCD order 102 heads S512
+//   0.94, 160 heads S199 0.91) and, at D = 64, of
 //   rows past 384 or past 7/4 blocks a CU (89 heads S512 1.08, 102 heads 0.93; 253 heads S256 1.07
 //   to 1.29, 179 heads 0.94).
 bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
@@ -722,7 +723,7 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (n <= ncu) return false;
   if (!a->causal) {
     if (n % 8 != 0 && n <= 2 * (int64_t)ncu && use_rows256(a, n_bh, ncu) && S > 192 * ((S + 255) / 256) &&
-        (a->D == 128 || S > 384 || 4 * n > 7 * (int64_t)ncu))
+        (a->D == 128 ? S <= 224 || S > 256 : S > 384 || 4 * n > 7 * (int64_t)ncu))
       return false;
     if (a->D == 64) return S <= 512 || (S <= 1024 && n >= 4 * (int64_t)ncu);
     return S <= (a->D == 96 ? 1024 : a->D == 128 ? 512 : 768);
