@@ -44,8 +44,8 @@ namespace ta {
 // bytes a key row, of the eight-wave kernel at head dim D: 128 keys, 64 at D = 256, so that
 // two stages of K and of V take 130 KiB of LDS there.  A cluster is then 16 QK^T and 16 P.V
 // MFMAs as at D = 128, with half the scores a lane, and is bound by its MFMAs and their LDS
-// operands (1 KiB each): bf16 B1 H8 S4096 non-causal 1080 TFLOP/s, causal 188 (four-wave
-// kernel) -> 87 us.
+// operands (1 KiB each): bf16 B1 H8 S4096 non-causal 1130 TFLOP/s (122 us), causal 197 (four-wave
+// kernel) -> 92 us, where the heaviest of its 256 blocks, one a CU, takes 64 steps of a mean 33.
 constexpr int pp_step_keys(int d) { return d == 256 ? kPPKeys / 2 : kPPKeys; }
 constexpr int pp_stage_bytes(int d) { return pp_step_keys(d) * 2 * d; }
 // LDS bytes from one 1 KiB chunk of a K stage to the next: at D = 256 (two rows a chunk) 32
@@ -730,11 +730,20 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
       }
     }
   };
+  // Where the key loop starts, to the 4 bytes modulo 32, is worth 1-2 % in these kernels, whatever
+  // the length of the prologue in front of it: D = 160 causal 24 heads S1536 bf16 28.9 -> 28.4 us,
+  // input-dtype D = 64 causal 32 heads S2819 bf16 0.995 of the time at an arbitrary place.
+  auto place_loop = [&]() {
+    if constexpr (D == 160 && CAUSAL && !SPLIT && TM == 128)
+      asm volatile(".p2align 5\ns_nop 0\ns_nop 0\ns_nop 0\ns_nop 0");
+    if constexpr (D == 64 && CAUSAL && LOWP && TM == 128) asm volatile(".p2align 5\ns_nop 0\ns_nop 0");
+  };
   using G0 = std::false_type;
   using G1 = std::integral_constant<bool, R256>;  // group 1's own load schedule (R256 only)
   if (grp == 0) {
     first();
     barrier();
+    place_loop();
     for (int t = t_beg; t < t_end; t += 2) {
       iter(t, std::integral_constant<int, 0>{}, G0{});
       if (t + 1 < t_end) iter(t + 1, std::integral_constant<int, 1>{}, G0{});
@@ -744,6 +753,7 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
     barrier();  // phase 0: group 0's S_0
     first();
     barrier();
+    place_loop();
     for (int t = t_beg; t < t_end; t += 2) {
       iter(t, std::integral_constant<int, 0>{}, G1{});
       if (t + 1 < t_end) iter(t + 1, std::integral_constant<int, 1>{}, G1{});
