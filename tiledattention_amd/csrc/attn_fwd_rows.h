@@ -14,10 +14,10 @@
 //   (attn_fwd_pp.hip).
 //
 // It runs the grids of short rows and many heads, where the eight-wave kernel's workgroup, one
-// a CU, spends as long on its prologue, pipeline fill and merge as on its keys.  B32 H12 S197
-// D64 fp16 non-causal 17.1 -> 12.9 us, B16 H16 S512 D64 bf16 31.3 -> 26, B64 H12 S128 D64 fp16
-// causal 20.1 -> 11.2, B8 H32 S320 D128 bf16 30.1 -> 25.8 (their 39, 67, 75 and 84 MB of q, k, v
-// and o take 7.4, 12.8, 14.4 and 16 us at a large copy's rate).  Long rows reach what the
+// a CU, spends as long on its prologue, pipeline fill and merge as on its keys.  Back-to-back
+// launches of both on one card: B32 H12 S197 D64 fp16 non-causal 16.0 -> 13.2 us, B16 H16 S512 D64
+// bf16 31.4 -> 25.7, B64 H12 S128 D64 fp16 causal 20.2 -> 11.1, B8 H32 S320 D128 bf16 31.3 -> 26.7
+// (their 39, 67, 75 and 84 MB of q, k, v and o take 7.4, 12.8, 14.4 and 16 us at a large copy's rate).  Long rows reach what the
 // eight-wave kernels do at D = 64 and less at 128 (B4 H16 S4096: 278 us against 265, 482 against
 // 427), and few blocks lose (B1 H8 S8192 D64 causal 102 against 76).  64 query rows a wave, which
 // halves the LDS operand reads, was not faster (12.4 -> 14.1, 24.3 -> 24.4 us), nor were eight
@@ -30,8 +30,8 @@
 //
 // Input-dtype accumulation (LOWP_TN): the same workgroups with the eight-wave kernel's two key
 // slices a row, both in one wave (even and odd tiles), so results and errors are the same to the
-// merge's last bit (2-norm 1e-5): C4's D = 64 shape, fp16 404 -> 362 us, bf16 402 -> 340;
-// B16 H16 S512 fp16 41 -> 29.  VALU-bound (84 % of cycles): per tile and lane 32 FMAs, 32
+// merge's last bit (2-norm 1e-5): B4 H16 S4096 D64 fp16 430 -> 369 us, bf16 430 -> 352;
+// B16 H16 S512 fp16 44 -> 30.  VALU-bound (84 % of cycles): per tile and lane 32 FMAs, 32
 // exponentials, 32 sums, 16 maxima, 16 packs, the rounding of O (48) and its rescale (32, three
 // tiles in five).  The rescale is a branch of its own in front of one rounding: a branch with a
 // rounding on either side kept a second copy of O alive (7-13 registers spilled at D = 64, over
