@@ -1,6 +1,6 @@
-"""Benchmark of the SDPA forward on one MI355X (the driver's bench contract).
+"""Benchmark of the SDPA forward on one MI355X.
 
-Headline workload (BASELINE.json north star): C3 at S=8192 - B=1, H=8, S=8192, D=128,
+Headline workload: C3 at S=8192 - B=1, H=8, S=8192, D=128,
 bf16, causal, seed 1234, default knobs.  A "step" is one forward over that batch with the
 inputs already resident in HBM.  Work per step is 4*B*H*S^2*D FLOPs halved for causal
 (137.4 GFLOP), so ``value`` is TFLOP/s.
@@ -17,7 +17,7 @@ measured, and with ``--detail-json FILE`` to that file, as one JSON record of th
 * ``cpu_baseline``: the reference's eager attention restated on the host CPU
   (oracle/eager.py, run_study.py:304-335) on a bounded sample of the same workload;
 * ``sweep``: the C3 sequence sweep S in {512..8192} (bf16);
-* ``blocks``: every other BASELINE.json configuration, each timed the same way (TFLOP/s,
+* ``blocks``: every other configuration of the reference study, each timed the same way (TFLOP/s,
   share of peak, algorithmic HBM GB/s, mean and p95 per call, the kernel the library
   launches): C2, the C4 tile x accumulation sweep (fp16/bf16, D 64/128), C5 and its outlier
   variant C5b; ``grid``, the metric's curves: B1 H8, S in {512..8192}, fp16 and bf16, causal
@@ -91,7 +91,7 @@ def _args():
     ap.add_argument("--seq", type=int, default=8192, help="sequence length of the headline workload")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-sweep", action="store_true")
-    ap.add_argument("--no-blocks", action="store_true", help="skip the other BASELINE configurations")
+    ap.add_argument("--no-blocks", action="store_true", help="skip the other configurations")
     ap.add_argument("--detail-json", default="", help="write the whole record (sweep, blocks) to this file")
     ap.add_argument("--only-block", default="", help="run only blocks whose name starts with this")
     ap.add_argument("--traffic-json", default=str(ROOT / "profiles" / "traffic.json"),
@@ -114,7 +114,7 @@ def make_inputs(shape, dtype: str, seed: int, *, scale_inputs: float = 1.0, outl
     """Seeded q, k, v (CPU tensors of ``dtype``): ``randn`` in fp32 from
     ``torch.Generator('cpu').manual_seed(seed)`` in the order q, k, v (run_study.py:526-529),
     times ``scale_inputs``; ``outlier_frac`` > 0 multiplies that fraction of k's entries,
-    chosen uniformly with ``outlier_seed``, by ``outlier_gain`` (BASELINE config C5b)."""
+    chosen uniformly with ``outlier_seed``, by ``outlier_gain`` (configuration C5b)."""
     import torch
 
     tdt = {"float16": torch.float16, "bfloat16": torch.bfloat16}[dtype]
@@ -131,7 +131,7 @@ def make_inputs(shape, dtype: str, seed: int, *, scale_inputs: float = 1.0, outl
 
 
 def flops_of(b: int, h: int, s: int, d: int, causal: bool) -> float:
-    """Work of one forward as BASELINE.json counts it: 4*B*H*S^2*D, halved when causal."""
+    """Work of one forward: 4*B*H*S^2*D, halved when causal."""
     f = 4.0 * b * h * s * s * d
     return f / 2.0 if causal else f
 
@@ -262,7 +262,7 @@ def clear_mantissa(t, keep_bits: int = 0):
 
 
 def run_blocks(dev, only: str = "") -> dict:
-    """Every BASELINE.json configuration beside the headline, timed like the sweep."""
+    """Every other configuration beside the headline, timed like the sweep."""
     import torch
 
     from tiledattention import sdpa
@@ -506,7 +506,7 @@ def main() -> int:
     args = _args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU only; --gpus {args.gpus} is not supported in this build "
-              "(every GPU box here has one GPU).", file=sys.stderr)
+              "(one GPU at a time).", file=sys.stderr)
         return 2
 
     import torch

@@ -5,7 +5,7 @@
  * Three restatements, all reading fp16/bf16 bit patterns and upcasting exactly:
  *
  *  ora_explicit_f32 / ora_explicit_f64
- *      The north-star oracle: explicit softmax(Q K^T * scale + mask) V with every operation
+ *      The explicit oracle: softmax(Q K^T * scale + mask) V with every operation
  *      in fp32 (or fp64), one query row at a time.  Mask: key j allowed for query i iff
  *      j <= i when causal (the reference's `row >= col`, flash_fwd.py:420-421).
  *

@@ -7,8 +7,8 @@ baseline; the operator in ``tiledattention`` never imports it and has no CPU fal
 Contents:
 
 * ``explicit_f32`` / ``explicit_f64`` - explicit softmax(QK^T*scale + mask)V, every step in
-  fp32 (fp64), from the upcast fp16/bf16 inputs: the correctness oracle named by the
-  north star.  C implementation in ``attention_oracle.c``.
+  fp32 (fp64), from the upcast fp16/bf16 inputs: the correctness oracle.
+  C implementation in ``attention_oracle.c``.
 * ``flash_tiled`` - restatement of the reference kernel's tiled online-softmax algorithm
   (src/tiledattention/kernels/flash_fwd.py:374-446, and :301-372 for accumulation in the
   input dtype), rounding to the input dtype exactly where the reference casts.
@@ -219,7 +219,7 @@ def to_bits(t) -> np.ndarray:
 # --------------------------------------------------------------------------- measurement
 
 def attention_forward_flops(*, b: int, h: int, s: int, d: int, causal: bool) -> float:
-    """Work of one forward as the north star counts it: 4*B*H*S^2*D, halved when causal."""
+    """Work of one forward: 4*B*H*S^2*D, halved when causal."""
     f = 4.0 * b * h * s * s * d
     return f / 2.0 if causal else f
 

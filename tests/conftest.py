@@ -52,7 +52,7 @@ def gpu_available() -> bool:
 
 @pytest.fixture
 def gpu():
-    """Skip unless a GPU is visible; on a GPU box the kernels must be built (fail loudly)."""
+    """Skip unless a GPU is visible; on a GPU machine the kernels must be built (fail loudly)."""
     if not gpu_available():
         pytest.skip("no GPU visible")
     from tiledattention import _runtime

@@ -4,7 +4,7 @@ Each fixture holds seeded inputs (fp16/bf16 bit patterns) and the explicit fp32 
 oracle outputs, computed by this repository's oracle (oracle/attention_oracle.c).  The
 reference holds no numeric fixtures of its own for this path (its only numeric check,
 tests/test_sdpa_correctness_small.py, draws inputs on the GPU at run time), so these pin
-the oracle's outputs against silent change and carry them to the GPU box.
+the oracle's outputs against silent change and carry them to GPU machines.
 
 Run from the repository root: ``python -m tests.golden.make_golden``.
 """

@@ -1,6 +1,6 @@
 """Helpers shared by the GPU parity tests: seeded inputs, oracle comparison, env knobs.
 
-Tolerances (max-abs against the explicit fp32 oracle, from the north star): 2e-3 for
+Tolerances (max-abs against the explicit fp32 oracle): 2e-3 for
 fp16, 1e-2 for bf16.  Input-dtype accumulation (TILEDATTN_ACCUM_MODE=fp16) rounds O to the
 input dtype after every key tile, as the reference does (flash_fwd.py:360-362); it is held
 to 2.5x those bounds against the fp32 oracle and to the input dtype's own rounding against

@@ -303,7 +303,7 @@ def test_zero_size_and_invalid_requests(lib):
 
 
 def test_policy_defaults_run_the_described_kernels(lib):
-    """The host policy's default tiles for the BASELINE configurations, through the library:
+    """The host policy's default tiles for the study's configurations, through the library:
     C1 64-row tile on the wide kernel (tail variant: S = 64 is not a whole 128-key step), C2
     (64, 64) non-causal and C3 S = 512 the wide kernel (32-row blocks in one round of the
     CUs), C3 S = 2048 the 64-row kernel (512 blocks of 32 rows would be two rounds), S = 4096

@@ -1,4 +1,4 @@
-"""Driver-facing entry points on the CPU: bench.py's one-GPU contract, __graft_entry__."""
+"""Entry points on the CPU: bench.py's one-GPU contract, __graft_entry__."""
 
 from __future__ import annotations
 

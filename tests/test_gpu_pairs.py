@@ -2,7 +2,7 @@
 j of a head, ``ta_fwd_args.sched`` 1 on grids of two or more workgroups per CU, or 3).
 
 Each block is computed exactly as in the one-block-per-workgroup grid, so the paired output
-must equal the unpaired one (TILEDATTN_SCHED=0) bit for bit, and meet the north-star bound
+must equal the unpaired one (TILEDATTN_SCHED=0) bit for bit, and meet the oracle tolerance
 against the fp32 oracle (sampled rows for the long sequences).  Every case names itself."""
 
 from __future__ import annotations

@@ -1,4 +1,4 @@
-"""GPU parity of the gfx950 SDPA forward against the CPU oracle, at every BASELINE config.
+"""GPU parity of the gfx950 SDPA forward against the CPU oracle, at every configuration of the study.
 
 Every case names itself on stdout before touching the GPU.  Inputs come from the CPU
 generator (oracle.make_inputs), so they are bit-identical to what the oracle sees.  Sizes
@@ -31,7 +31,7 @@ pytestmark = pytest.mark.gpu
 TILES = [(64, 64), (64, 128), (128, 64), (128, 128)]
 
 
-# ---------------------------------------------------------------- BASELINE configs
+# ---------------------------------------------------------------- the study's configurations
 
 def test_c1_example_workload_all_tiles(gpu):
     """C1: B1 H2 S64 D64 fp16 causal, seed 0 (the reference's example.py:19-24 workload)."""

@@ -1,8 +1,8 @@
 """Seeded randomised GPU parity: 40 configurations drawn from one fixed generator, each
 against the explicit fp32 attention of the CPU oracle.
 
-Draws whose logits spread like the north star's (standard deviation of scale * q.k up to
-6) are held to the north-star tolerance (2e-3 fp16, 1e-2 bf16; the input-dtype
+Draws whose logits spread like N(0, 1) inputs' (standard deviation of scale * q.k up to
+6) are held to the oracle tolerance (2e-3 fp16, 1e-2 bf16; the input-dtype
 accumulation bound for ``ACCUM_MODE=fp16``), scaled by the input magnitude.  Sharper draws
 (inputs x2 with scale 0.3: a nearly one-hot softmax) are dominated by the rounding of P to
 the input dtype, which the reference's algorithm performs too: with unit roundoff u

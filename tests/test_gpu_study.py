@@ -58,7 +58,7 @@ def test_harness_methods_compute_attention(gpu, dtype, causal):
     """Every method the study times computes the attention it is timed for: the inputs the
     harness generates (torch.manual_seed(1234), N(0,1) on the GPU, run_study.py:526-529),
     each method's output against the explicit fp32 oracle on the same values.  The
-    ``tiledattention`` rows meet the north-star bound; PyTorch's own paths 5e-2 (the eager
+    ``tiledattention`` rows meet the oracle tolerance; PyTorch's own paths 5e-2 (the eager
     path rounds its scores to the input dtype; the check is that they are attention, which
     a transposed operand, a dropped scale or a shifted mask would miss by far more)."""
     import torch

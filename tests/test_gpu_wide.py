@@ -7,7 +7,7 @@ causal and not, ragged S (rows and keys past S: the tail variants, including S a
 32 but not of a wave's 64 keys), both dtypes and head dims, head dims padded in place
 (d_real), strided views and a custom scale.  Each case first checks that the library
 describes the wide kernel for it (``ta_describe_launch``), names itself before touching the
-GPU, and compares the whole output at the north-star bound.
+GPU, and compares the whole output at the oracle tolerance.
 """
 
 from __future__ import annotations
@@ -102,7 +102,7 @@ _WIDE_CASES = [_wide_draw(r) for r in [random.Random(20261202)] for _ in range(2
 @pytest.mark.parametrize("case", _WIDE_CASES, ids=[f"w{i}" for i in range(len(_WIDE_CASES))])
 def test_wide_randomized(gpu, case):
     """Seeded random configurations inside the wide rule against the explicit fp32 oracle, at
-    the north-star tolerance scaled by the input magnitude; draws with a sharp softmax
+    the oracle tolerance scaled by the input magnitude; draws with a sharp softmax
     (logit spread above 6) at the P-rounding bound 3 u max|v| instead (the reasoning of
     tests/test_gpu_randomized.py)."""
     import math

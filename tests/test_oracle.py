@@ -2,7 +2,7 @@
 
 What pins what:
 
-* ``explicit_f32`` (the north-star oracle):
+* ``explicit_f32`` (the explicit oracle):
   - against ``explicit_f64`` (same algorithm, another precision),
   - against ``torch.nn.functional.scaled_dot_product_attention`` in fp32 on the CPU
     (a library routine),

@@ -3,7 +3,7 @@
 It must give exactly what ta_sdpa_fwd_split gives with a caller-owned workspace (the same
 kernels; only the workspace's address differs), on two calls in a row whose second is
 smaller (the static array keeps the first call's partials), for chunk lengths and the
-paired split, and meet the north-star bound against the fp32 oracle.  Torch only allocates the tensors and provides the stream."""
+paired split, and meet the oracle tolerance against the fp32 oracle.  Torch only allocates the tensors and provides the stream."""
 
 from __future__ import annotations
 
