@@ -131,6 +131,24 @@ def test_rows_falling_maxima(gpu, dtype):
     check_close(_run((q, k, v), True), ref, dtype, tol=3 * u * float(v.float().abs().max()), what="rows falling maxima")
 
 
+@pytest.mark.parametrize("causal", [False, True])
+def test_rows_large_values_with_falling_maxima(gpu, causal):
+    """Values near the top of bf16's range, and keys whose tiles' maxima fall: what is kept while
+    the reference point follows them stays finite."""
+    import torch
+
+    q, k, v = inputs((33, 8, 192, 64), "bfloat16", 84)
+    step = torch.tensor([4.0, 2.0, 0.0])[torch.arange(192) // 64]
+    q = (q.float().abs() * 0.25 + 0.5).to(q.dtype)
+    k = (0.25 * k.float() + step[None, None, :, None]).to(k.dtype)
+    v = (v.float().clamp(-2.0, 2.0) * 2.0 ** 118).to(v.dtype)
+    ref = oracle_f32(q, k, v, causal=causal) * 2.0 ** -118
+    assert np.isfinite(ref).all()
+    got = _run((q, k, v), causal) * np.float32(2.0 ** -118)
+    # P's rounding u = 2^-8, as above
+    check_close(got, ref, "bfloat16", tol=3 * 2.0 ** -8 * 2.0, what=f"rows large values causal={causal}")
+
+
 @pytest.mark.parametrize("value", [float("nan"), float("-inf")])
 def test_rows_nonfinite_keys(gpu, value):
     """A NaN key poisons every row of its head; a key whose scores are -inf or +inf by the

@@ -50,9 +50,8 @@ namespace ta {
 
 constexpr int kRowsKeys = 64;  // keys per tile
 constexpr int kRowsWaves = 4;
-constexpr int kRowsExact = 3;  // tiles with an exact max of their own
-constexpr float kRowsDrop = 7.0f;  // two drops stay below the lazy rule's 2^15
-static_assert((kRowsExact - 1) * kRowsDrop <= kRescaleLog2, "growth of O and l");
+constexpr int kRowsExact = 3;  // tiles whose largest P is exact
+constexpr float kRowsFar = 32.0f;  // a tile that far (log2) below the point keeps the point
 
 // p.n_qblk = ceil(S / 128).
 template <int DT, int D, bool CAUSAL, bool TAIL, int LOWP_TN = 0>
@@ -100,7 +99,6 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
   const int v_rb = (int)p.v_ss * 2;
   const int d_real = p.d_real;
   const float c = p.scale_log2;
-  const float drop = kRowsDrop * __builtin_amdgcn_rcpf(c);  // in raw score units
 
   const int q0 = wi.qt * TM;
   const int wq0 = q0 + 32 * wave;
@@ -281,38 +279,40 @@ __device__ __forceinline__ void attn_fwd_rows_body(const FwdParams& p) {
       }
       return (l4[0] + l4[1]) + (l4[2] + l4[3]);
     };
-    // Reference point of P: over the first kRowsExact tiles each tile's own exact max (O and l
-    // are zero at the first: nothing to rescale), so that a row's largest P of every such tile is
-    // exactly 1 and carries no rounding, as in the eight-wave kernel, whose two key halves have a
-    // max each; from then on the lazy rule of that kernel (the max is reduced only where some
-    // lane's sum of P reaches the bound).  A tile whose max lies more than kRowsDrop (log2 units)
-    // below the point so far takes that much less instead, which bounds how far O and l grow.
+    // Reference point of P: over the first kRowsExact tiles (O and l are zero at the first: nothing
+    // to rescale) every tile's largest P is an exact power of two and carries no rounding: the
+    // tile's own max where that is above the point so far, else whole log2 units above that max and
+    // less than one below the point, so that O and l less than double.  That is as exact as the
+    // eight-wave kernel, whose two key halves have a max each.  From then on the lazy rule of that
+    // kernel (the max is reduced only where some lane's sum of P reaches the bound).
     // Against 64 bits, the eight-wave kernel's error = 1 (B H 264-384, N(0, 1), both dtypes):
     // with the running max instead S96 to S113 1.014-1.016, S128 1.013, causal to S200
     // 1.002-1.003; every further exact tile costs 1 % of the time.
+    // (m_run is in log2 units here, score times c.)
     if constexpr (!LOWP) {
       if (t < kRowsExact) {
-        const float m_new = vmax(m_run - drop, row_max());
+        const float mx = vmax(row_max() * c, m_run - kRowsFar);
+        const float m_new = mx + vmax(__builtin_floorf(m_run - mx), 0.0f);
         if (t > 0 && __ballot(!(m_new == m_run))) {
-          const float alpha = fast_exp2((m_run - m_new) * c);
+          const float alpha = fast_exp2(m_run - m_new);
 #pragma unroll
           for (int db = 0; db < DB; ++db) o_acc[db] *= alpha;
           l_part *= alpha;
         }
         m_run = m_new;
       }
-      float l_step = make_p(m_run * c);
+      float l_step = make_p(m_run);
       if (t >= kRowsExact && __ballot(!(l_step < kRescaleBound))) {
-        const float mx = row_max();
-        const bool need = (mx - m_run) * c > kRescaleLog2;
+        const float mx = row_max() * c;
+        const bool need = mx - m_run > kRescaleLog2;
         if (__ballot(need)) {
           const float m_new = need ? mx : m_run;
-          const float alpha = fast_exp2((m_run - m_new) * c);
+          const float alpha = fast_exp2(m_run - m_new);
           m_run = m_new;
 #pragma unroll
           for (int db = 0; db < DB; ++db) o_acc[db] *= alpha;
           l_part *= alpha;
-          l_step = make_p(m_run * c);
+          l_step = make_p(m_run);
         }
       }
       l_part += l_step;
