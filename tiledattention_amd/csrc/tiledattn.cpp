@@ -720,6 +720,9 @@ KernelId pp_d256_kernel_id(int dtype, int causal, int tail) {
 //   0.94, 160 heads S199 0.91) and, at D = 64, of
 //   rows past 384 or past 7/4 blocks a CU (89 heads S512 1.08, 102 heads 0.93; 253 heads S256 1.07
 //   to 1.29, 179 heads 0.94).
+// Both dtypes swept against the eight-wave kernels (3000 grids, D 64-160): what is left of losses
+// is 1-3 % (128 heads S512 D64 causal bf16; 72 and 80 heads S455-512 non-causal) and 1-7 % at D =
+// 128 causal S 609-640 from 2.5 blocks a CU where the XCDs cannot take whole heads.
 bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (!eight_wave(a->tile_m, a->tile_n, a->accum, a->D) || a->sched == 3 || ncu <= 0) return false;
   const int64_t S = a->S, n = n_bh * n_qblk;
