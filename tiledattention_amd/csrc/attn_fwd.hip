@@ -219,8 +219,11 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
   // RPC g + l / CPR, so it loads logical chunk (l % CPR) ^ swz(row) of that row.  Rows
   // RPC NW i apart: K's swizzle repeats every 16 rows (KP distinct per-lane offsets, the
   // rest a uniform row step), V's every 4 (one offset).  Rows past S are outside the
-  // tile's buffer resource and read as zero; the row steps go into the per-lane offset, as a
-  // load's scalar offset is no part of its documented range check.
+  // tile's buffer resource and read as zero.  A load's scalar offset is no part of its documented
+  // range check, so the row steps go elsewhere: with fp32 accumulation into resources that start
+  // there (in the per-lane offset their registers cost 3-7 %: B1 H8 S4096 causal bf16 182 us here,
+  // 196 there), with input-dtype accumulation, which has registers left, into the per-lane offset
+  // (1 % faster there).
   constexpr int RPC = 1024 / (2 * D);
   constexpr int NCH = TN * 2 * D / 1024;
   constexpr int NLW = NCH / NW;  // loads per wave per tensor per tile
@@ -243,25 +246,24 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
     }
     dm_v = row0 * v_rb + ((pc ^ L::swz_v(row0)) << 4);
   }
+  // One chunk of a tile that starts at `tile`: `step` rows on from the lane's offset `vo`.
+  auto dma_chunk = [&](const uint16_t* tile, int rows, int rb, int vo, int step, char* chunk) {
+    const __amdgpu_buffer_rsrc_t r =
+        LOWP ? row_rsrc(tile, rows, rb) : row_rsrc((const char*)tile + step * rb, rows - step, rb);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)chunk, 16,
+                                             LOWP ? vo + step * rb : vo, 0, 0, 0);
+  };
   auto dma_k = [&](int kt, int stage) {
-    const __amdgpu_buffer_rsrc_t kr = row_rsrc(kp + (int64_t)kt * TN * p.k_ss, S - kt * TN, k_rb);
     char* base = smem + stage * STAGE;
 #pragma unroll
-    for (int i = 0; i < NLW; ++i) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          kr, (__attribute__((address_space(3))) void*)(base + (wave + NW * i) * 1024), 16,
-          dm_k[i % KP] + (i / KP) * 16 * k_rb, 0, 0, 0);
-    }
+    for (int i = 0; i < NLW; ++i)
+      dma_chunk(kp + (int64_t)kt * TN * p.k_ss, S - kt * TN, k_rb, dm_k[i % KP], (i / KP) * 16, base + (wave + NW * i) * 1024);
   };
   auto dma_v = [&](int kt, int stage) {
-    const __amdgpu_buffer_rsrc_t vr = row_rsrc(vp + (int64_t)kt * TN * p.v_ss, S - kt * TN, v_rb);
     char* base = smem + stage * STAGE + K_BYTES;
 #pragma unroll
-    for (int i = 0; i < NLW; ++i) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          vr, (__attribute__((address_space(3))) void*)(base + (wave + NW * i) * 1024), 16,
-          dm_v + i * RSTEP * v_rb, 0, 0, 0);
-    }
+    for (int i = 0; i < NLW; ++i)
+      dma_chunk(vp + (int64_t)kt * TN * p.v_ss, S - kt * TN, v_rb, dm_v, i * RSTEP, base + (wave + NW * i) * 1024);
   };
 
   // ---- per-lane LDS read offsets --------------------------------------------------------

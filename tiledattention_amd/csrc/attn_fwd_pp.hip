@@ -44,8 +44,8 @@ namespace ta {
 // bytes a key row, of the eight-wave kernel at head dim D: 128 keys, 64 at D = 256, so that
 // two stages of K and of V take 130 KiB of LDS there.  A cluster is then 16 QK^T and 16 P.V
 // MFMAs as at D = 128, with half the scores a lane, and is bound by its MFMAs and their LDS
-// operands (1 KiB each): bf16 B1 H8 S4096 non-causal 1130 TFLOP/s (122 us), causal 197 (four-wave
-// kernel) -> 92 us, where the heaviest of its 256 blocks, one a CU, takes 64 steps of a mean 33.
+// operands (1 KiB each): bf16 B1 H8 S4096 non-causal 1184 TFLOP/s (116 us), causal 181 (four-wave
+// kernel) -> 90 us, where the heaviest of its 256 blocks, one a CU, takes 64 steps of a mean 33.
 constexpr int pp_step_keys(int d) { return d == 256 ? kPPKeys / 2 : kPPKeys; }
 constexpr int pp_stage_bytes(int d) { return pp_step_keys(d) * 2 * d; }
 // LDS bytes from one 1 KiB chunk of a K stage to the next: at D = 256 (two rows a chunk) 32
@@ -253,7 +253,9 @@ __device__ __forceinline__ void attn_fwd_pp_block(const FwdParams& p, const Work
   const int qvo = 8 * lck < d_real ? ld_row * q_rb + (lck << 4) : kZeroChunk;
   const int tqvo = DA + 8 * tl_lck < d_real ? tl_row * q_rb + 2 * DA + (tl_lck << 4) : kZeroChunk;
   // A chunk's row step from the wave's first goes into the per-lane offset: a load's scalar
-  // offset is no part of its documented range check, which zeroes rows past S.
+  // offset is no part of its documented range check, which zeroes rows past S.  (At D = 256, where
+  // registers are short, a resource for each step instead spills scalar ones: B1 H8 S4096 causal
+  // bf16 112 us against 89.)
   constexpr int KCH = pp_k_chunk(D);
   auto dma = [&](const uint16_t* gbase, int64_t row_stride, int rb, int vo, int tvo, int t, char* stage,
                  int chunk_bytes) {

@@ -656,10 +656,10 @@ bool use_rows256(const ta_fwd_args* a, int64_t n_bh, int ncu) {
 
 // Whether a whole-row launch at D = 256 runs the eight-wave kernel (ta_fwd_pp_*_d256_*; steps
 // of 64 keys): fp32 accumulation, 128-row tiles, rows of more than one key step (bf16, four-wave
-// kernel -> this one: B1 H8 S4096 causal 197 -> 92 us, non-causal 195 -> 121, B1 H2 S512 causal
-// 31.4 -> 17.9, B4 H16 S128 causal 15.0 -> 12.7; at one step they are even, B1 H8 S64 9.7 -> 10.1,
+// kernel -> this one: B1 H8 S4096 causal 181 -> 90 us, non-causal 173 -> 116, B1 H2 S512 causal
+// 29.4 -> 17.8, B4 H16 S128 causal 14.6 -> 12.7; at one step they are even, B1 H8 S64 9.7 -> 10.1,
 // B4 H32 S64 9.7 -> 9.5).  One head of at most four blocks stays on the four-wave kernel although
-// this one is faster there too (causal B1 H1 S65 11.7 -> 10.9, S256 19.9 -> 13.1, S512 31.4 -> 17.6):
+// this one is faster there too (causal B1 H1 S65 11.6 -> 10.9, S256 19.0 -> 13.2, S512 29.7 -> 17.8):
 // the table of one small head's launch per configuration names the four-wave kernel
 // (test_describe.py, test_whole_row_kernel_per_configuration), so the line can only move with that
 // table.  And so does a grid whose 512-thread workgroups would pass the dispatch packet's 2^32
