@@ -218,7 +218,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
   // each); wave w fills chunks g = w + NW i, lane l writing physical chunk l % CPR of row
   // RPC g + l / CPR, so it loads logical chunk (l % CPR) ^ swz(row) of that row.  Rows
   // RPC NW i apart: K's swizzle repeats every 16 rows (KP distinct per-lane offsets, the
-  // rest a uniform row step), V's every 4 (one offset).  Rows past S are outside the
+  // rest a uniform row step), V's every 4 (KP offsets as well).  Rows past S are outside the
   // tile's buffer resource and read as zero.  A load's scalar offset is no part of its documented
   // range check, so the row steps go elsewhere: with fp32 accumulation into resources that start
   // there (in the per-lane offset their registers cost 3-7 %: B1 H8 S4096 causal bf16 182 us here,
@@ -235,7 +235,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
   constexpr int KP = DMA ? 16 / RSTEP : 1;
   static_assert(!DMA || (NCH % NW == 0 && 16 % RSTEP == 0 && RSTEP % 4 == 0), "DMA tiling");
   int dm_k[KP];
-  int dm_v = 0;
+  int dm_v[KP];
   if constexpr (DMA) {
     const int row0 = RPC * wave + lane / CPR;
     const int pc = lane % CPR;
@@ -244,7 +244,8 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
       const int row = row0 + RSTEP * j;
       dm_k[j] = row * k_rb + ((pc ^ L::swz_k(row)) << 4);
     }
-    dm_v = row0 * v_rb + ((pc ^ L::swz_v(row0)) << 4);
+#pragma unroll
+    for (int j = 0; j < KP; ++j) dm_v[j] = (row0 + RSTEP * j) * v_rb + ((pc ^ L::swz_v(row0)) << 4);
   }
   // One chunk of a tile that starts at `tile`: `step` rows on from the lane's offset `vo`.
   auto dma_chunk = [&](const uint16_t* tile, int rows, int rb, int vo, int step, char* chunk) {
@@ -263,7 +264,7 @@ __device__ __forceinline__ void attn_fwd_body(const FwdParams& p) {
     char* base = smem + stage * STAGE + K_BYTES;
 #pragma unroll
     for (int i = 0; i < NLW; ++i)
-      dma_chunk(vp + (int64_t)kt * TN * p.v_ss, S - kt * TN, v_rb, dm_v, i * RSTEP, base + (wave + NW * i) * 1024);
+      dma_chunk(vp + (int64_t)kt * TN * p.v_ss, S - kt * TN, v_rb, dm_v[i % KP], (i / KP) * 16, base + (wave + NW * i) * 1024);
   };
 
   // ---- per-lane LDS read offsets --------------------------------------------------------
