@@ -436,15 +436,22 @@ def test_small_workgroup_rule_input_dtype_near_one_block_a_cu(lib, d, tn, h, s, 
 # of pairs, the eight-wave kernels keep it.
 @pytest.mark.parametrize("d,causal,h,s,rows", [
     (64, False, 65, 512, False), (64, False, 66, 512, True), (64, False, 89, 449, False), (64, False, 102, 512, True),
-    (64, False, 129, 512, True), (64, False, 179, 256, True), (64, False, 253, 256, False), (64, False, 89, 384, True),
+    (64, False, 129, 512, True), (64, False, 179, 256, True), (64, False, 253, 256, False), (64, False, 253, 245, True),
+    (64, False, 89, 440, True), (64, False, 121, 512, True), (128, False, 71, 405, False), (128, False, 121, 405, True),
+    (128, False, 89, 512, False), (128, False, 121, 512, False), (128, False, 179, 224, False),
+    (128, False, 221, 224, True), (64, False, 89, 384, True),
     (128, False, 65, 512, False), (128, False, 102, 512, True), (128, False, 179, 199, False), (128, False, 221, 243, True),
     (128, False, 160, 199, True), (128, False, 179, 192, True), (128, False, 100, 330, True), (128, False, 257, 256, True),
     (64, True, 58, 1152, False), (64, True, 71, 1152, True), (64, True, 58, 1024, False), (96, True, 58, 1152, False),
-    (96, True, 57, 1088, True), (96, True, 57, 1089, False), (96, True, 71, 1152, True), (96, True, 53, 1536, True),
+    (96, True, 57, 1088, True), (96, True, 57, 1089, False), (96, True, 52, 1280, True),
+    (64, True, 43, 1536, True), (96, True, 129, 1472, True), (96, True, 86, 1536, True), (96, True, 71, 1152, True),
+    (96, True, 53, 1536, True),
     (96, True, 67, 1536, False), (64, True, 67, 1536, True),
     (128, True, 105, 576, True), (128, True, 105, 640, False), (128, True, 105, 609, False), (128, True, 107, 711, True),
-    (128, True, 107, 736, True), (128, True, 107, 768, False),
-    (160, True, 52, 640, False), (160, True, 58, 640, True), (160, True, 65, 512, True),
+    (128, True, 107, 736, True), (128, True, 107, 768, False), (128, True, 127, 768, False),
+    (128, True, 278, 768, False), (128, True, 278, 736, True),
+    (128, True, 118, 640, True),
+    (160, True, 52, 640, False), (160, True, 52, 580, True), (160, True, 54, 640, True), (160, True, 65, 512, True),
 ])
 def test_small_workgroup_rule_without_xcd_order(lib, d, causal, h, s, rows):
     desc = _d(lib, B=1, H=h, S=s, D=d, causal=causal, tile_m=128, sched=1)

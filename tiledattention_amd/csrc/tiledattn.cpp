@@ -707,36 +707,40 @@ KernelId pp_d256_kernel_id(int dtype, int causal, int tail) {
 // * causal otherwise: where the pairs of a grid of two blocks a CU or more fill one round of
 //   the CUs only up to S = 384 (D = 64 S512 128 heads 12.8 -> 13.2); else
 //   D = 64 and 96 up to 768, 1024 past four blocks a CU, and where the pairs' last round is short
-//   1536, past 1024 from 2.25 blocks a CU (58 heads S1152 D64 25.4 -> 26.3, D96 32.2 -> 34.2; 71
-//   heads 0.94 of the time), at D = 96 up to three (67 heads S1536 52.0 -> 56.1, 53 heads 0.94);
-//   D = 128 up to 512, past two blocks a CU 640 and, where the pairs' last round is short, 768, both
-//   only with 32 rows or more missing from the last block, which the small workgroups skip (107
-//   heads S711 0.96, S768 36.2 -> 37.1; 110 heads S640 29.5 -> 30.6), or up to 640 from 2.5 blocks;
-//   D = 160 up to 512, 640 from 9/8 blocks a CU (52 heads 23.3 -> 24.2);
+//   1536, but for heads of nine blocks below 2.25 blocks a CU with fewer than 64 rows missing from
+//   the last one, which the small workgroups skip (58 heads S1152 D64 25.4 -> 26.3, D96 32.2 -> 34.2;
+//   71 heads 0.94 of the time, 57 heads S1038 D96 0.86, 52 heads S1280 0.76), and at D = 96 S 1473 to
+//   1536 between 3 and 3.5 (67 heads S1536 52.0 -> 56.1; 53 heads 0.94, 86 heads 0.74);
+//   D = 128 up to 512, past two blocks a CU 640 with 32 rows or more missing from the last block, and
+//   from 2.25 all (110 heads S640 29.5 -> 30.6, 118 heads 0.97); where the pairs' last round is short
+//   768 with 32 rows missing (107 heads S711 0.96, S768 36.2 -> 37.1, on another card 1.06-1.09);
+//   D = 160 up to 640, but for full last blocks within 1/32 of one block a CU (52 heads S640 23.3 ->
+//   24.2, S580 0.98; 54 heads S640 0.97);
 // * non-causal grids that the XCDs cannot share evenly (n not a multiple of 8: both kernels then
-//   take heads in plain order, which costs the small workgroups more), one round of 256-row blocks
-//   whose rows are more than three quarters real: those at D = 128, but for rows of 225 to 256 (89
-//   heads S512 1.05 of the time, 179 heads S199 1.06, 221 heads S243 0.95; in XCD order 102 heads S512
-//   0.94, 160 heads S199 0.91) and, at D = 64, of
-//   rows past 384 or past 7/4 blocks a CU (89 heads S512 1.08, 102 heads 0.93; 253 heads S256 1.07
-//   to 1.29, 179 heads 0.94).
-// Both dtypes swept against the eight-wave kernels (3000 grids, D 64-160): what is left of losses
-// is 1-3 % (128 heads S512 D64 causal bf16; 72 and 80 heads S455-512 non-causal) and 1-7 % at D =
-// 128 causal S 609-640 from 2.5 blocks a CU where the XCDs cannot take whole heads.
+//   take heads in plain order, which costs the small workgroups more) and that are one round of
+//   256-row blocks.  D = 64: S past 448 up to 13/8 blocks a CU (71 heads S449 1.05 and S512 1.09 of the
+//   time, S440 0.93; 121 heads S512 0.98; in XCD order 102 heads S512 0.93), and 249 to 256 past 7/4
+//   (253 heads S256 1.02 to 1.29, S245 0.89).  D = 128: S 193 to 208, a fourth key tile for a few keys
+//   (179 heads S199 1.06; in XCD order 160 heads 0.91), to 224 and past 384 up to 3/2 (179 heads S215
+//   1.02, 71 heads S405 1.04; 221 heads S224 0.97, 115 heads S405 0.97), and past 448 (89 heads S512
+//   1.05, 121 heads 1.00 to 1.05).
+// Both dtypes swept against the eight-wave kernels (6000 grids, D 64-160).  The two kernels' times
+// differ from card to card by up to 7 % of one another, so the lines are no finer than that.
 bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
   if (!eight_wave(a->tile_m, a->tile_n, a->accum, a->D) || a->sched == 3 || ncu <= 0) return false;
-  const int64_t S = a->S, n = n_bh * n_qblk;
-  if (n <= ncu) return false;
+  const int64_t S = a->S, n = n_bh * n_qblk, cu = ncu;
+  if (n <= cu) return false;
   if (!a->causal) {
-    if (n % 8 != 0 && n <= 2 * (int64_t)ncu && use_rows256(a, n_bh, ncu) && S > 192 * ((S + 255) / 256) &&
-        (a->D == 128 ? S <= 224 || S > 256 : S > 384 || 4 * n > 7 * (int64_t)ncu))
-      return false;
-    if (a->D == 64) return S <= 512 || (S <= 1024 && n >= 4 * (int64_t)ncu);
+    if (n % 8 != 0 && n <= 2 * cu && use_rows256(a, n_bh, ncu)) {
+      if (a->D == 64 && ((S > 448 && 8 * n <= 13 * cu) || (S > 248 && S <= 256 && 4 * n > 7 * cu))) return false;
+      if (a->D == 128 && ((S > 192 && S <= 208) || (((S > 192 && S <= 224) || S > 384) && 2 * n <= 3 * cu) || S > 448))
+        return false;
+    }
+    if (a->D == 64) return S <= 512 || (S <= 1024 && n >= 4 * cu);
     return S <= (a->D == 96 ? 1024 : a->D == 128 ? 512 : 768);
   }
   if (S <= 384) return true;
   if (n_bh % 8 == 0 && a->sched == 1) {
-    const int64_t cu = ncu;
     const bool n225 = 4 * n >= 9 * cu, n375 = 4 * n >= 15 * cu;
     if (a->D == 160) return S <= 512 || (S <= 768 && 2 * n >= 3 * cu) || (S <= 1024 && n > 2 * cu) || (S <= 1536 && n >= 3 * cu);
     if (a->D == 128) return (S <= 448 && 2 * n <= 3 * cu) || (S <= 1024 && n > 2 * cu);
@@ -744,18 +748,18 @@ bool use_rows(const ta_fwd_args* a, int64_t n_bh, int64_t n_qblk, int ncu) {
     if (S <= 1280) return S <= 768 || (S <= 1024 && n >= 2 * cu) || n225;
     return (n_qblk % 2 == 0 || n > 4 * cu || !pairs_fill(n_bh, n_qblk, ncu)) && ((S <= 1536 && n225) || (S <= 3072 && n375));
   }
-  const int64_t cu = ncu;
-  if (a->D == 160) return S <= 512 || (S <= 640 && 8 * n >= 9 * cu);
-  const bool paired = n >= 2 * (int64_t)ncu;
+  const int64_t missing = 128 * n_qblk - S;  // rows of the last block
+  if (a->D == 160) return S <= 512 || (S <= 640 && (32 * n >= 33 * cu || missing >= 32));
+  const bool paired = n >= 2 * cu;
   const bool full = pairs_fill(n_bh, n_qblk, ncu);
   if (paired && full && n_bh * ((n_qblk + 1) / 2) <= ncu) return false;
   if (a->D == 128) {
-    const bool short_last = paired && 128 * n_qblk - S >= 32;
-    return S <= 512 || (S <= 640 && (short_last || 2 * n >= 5 * cu)) || (S <= 768 && short_last && !full);
+    if (S <= 512 || !paired) return S <= 512;
+    return S <= 640 ? missing >= 32 || 4 * n >= 9 * cu : S <= 768 && !full && missing >= 32;
   }
   if (S <= 768 || (S <= 1024 && n > 4 * cu)) return true;
-  if (S > 1536 || !paired || full) return false;
-  return S <= 1024 || ((4 * n >= 9 * cu || 128 * n_qblk - S >= 64) && (a->D == 64 || n <= 3 * cu));
+  if (S > 1536 || !paired || full || (S > 1024 && S <= 1152 && 4 * n < 9 * cu && missing < 64)) return false;
+  return a->D == 64 || S <= 1472 || n <= 3 * cu || 2 * n > 7 * cu;
 }
 
 // Whether input-dtype accumulation on a 128-row tile runs the small-workgroup kernel
